@@ -12,6 +12,7 @@
 //   * one symmetric two-grid cycle on S: pre-smooth W, exact coarse correction on
 //     aggregates (dense inverse), post-smooth W.
 // Every reduction runs in a fixed order: results are bitwise reproducible.
+#include <algorithm>
 #include <vector>
 
 #include "nfx_common.h"
@@ -240,14 +241,39 @@ __global__ void k_gnn_heads(int E, const int32_t* __restrict__ nbr, const float*
 }
 
 // ---------------------------------------------------------------------------
-// Backward (FP32). Weight-gradient partials per block, summed in block order.
+// Backward (FP32). Weight-gradient partials per block, summed in a fixed order.
 // ---------------------------------------------------------------------------
-constexpr int kBwdBlocks = 256;
-constexpr int kHeadPartial = 2 * kW + 2;            // ud, ue, cd, ce
+// Rows of 64 channels are read 16 bytes a lane; the types carry the element's alignment
+// only (the hardware takes an unaligned global access), so any base pointer is allowed.
+typedef float f4u_t __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t h8u_t __attribute__((ext_vector_type(4), aligned(2)));  // 8 bf16
+
+__device__ __forceinline__ void unpack8(const h8u_t& v, float (&o)[8]) {
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    o[2 * t] = __uint_as_float(v[t] << 16);
+    o[2 * t + 1] = __uint_as_float(v[t] & 0xFFFF0000u);
+  }
+}
+
+__device__ __forceinline__ float4_t mfma_f32_4(float a, float b, float4_t c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+// Most blocks (partial rows) of each kernel: the weight-gradient partials of a layer are 33 KB
+// a block, written and read once, so the layer kernel takes one block per 64-node tile only up
+// to two blocks per CU.
+constexpr int kBwdBlocks = 512;
+constexpr int kHeadBlocks = 1024;
+constexpr int kInBlocks = 512;
+constexpr int kHeadPartial = 2 * kW + 2;            // ud, cd, ue, ce (parameter order)
 constexpr int kLayerPartial = 2 * kW * kW + kW;     // Wh, Wm, b
 constexpr int kInPartial = kIn * kW + kW;           // W0, b0
 
-// dh_p = gN_p ud + (sum_j a_pj gE_pj) ue; partials of ud, ue, cd, ce.
+// dh_p = gN_p ud + (sum_j a_pj gE_pj) ue; partials of ud, cd, ue, ce. Bound by the gathers of
+// the neighbours' rows: 8 lanes share a node (8 channels, 16 bytes each), so a wave has 40 row
+// loads in flight, and E / 32 blocks fill the chip (24,576 nodes: 78 us with one thread per
+// channel walking 64 nodes on 96 blocks, 8.4 us now).
 __global__ __launch_bounds__(256) void k_heads_bwd(int E, const int32_t* __restrict__ nbr,
                                                    const float* __restrict__ a,
                                                    const uint16_t* __restrict__ th16,
@@ -257,154 +283,294 @@ __global__ __launch_bounds__(256) void k_heads_bwd(int E, const int32_t* __restr
                                                    const float* __restrict__ gam_o,
                                                    float* __restrict__ dh,
                                                    float* __restrict__ partial) {
-  __shared__ float sGn[256], sAg[256][4];
-  __shared__ int sQ[256][4];
-  const int tid = threadIdx.x;
-  const int c = tid & 63, grp = tid >> 6;
-  float pud = 0.f, pue = 0.f, pcd = 0.f, pce = 0.f;
-  for (int64_t t0 = (int64_t)blockIdx.x * 256; t0 < E; t0 += (int64_t)gridDim.x * 256) {
-    const int64_t p = t0 + tid;
-    float gn = 0.f, agsum = 0.f;
-    float ag[4] = {0.f, 0.f, 0.f, 0.f};
-    int qq[4] = {-1, -1, -1, -1};
-    if (p < E) {
-      const double dp = sdiag[p];
-      gn = float(gam_d[p] / dp);
-      for (int j = 0; j < 4; ++j) {
-        const int q = nbr[4 * p + j];
-        qq[j] = q;
-        if (q < 0) continue;
-        const float ge = float(gam_o[4 * p + j] / sqrt(dp * sdiag[q]));
-        ag[j] = a[4 * p + j] * ge;
-        agsum += ag[j];
-      }
-    }
-    sGn[tid] = gn;
-    for (int j = 0; j < 4; ++j) {
-      sAg[tid][j] = ag[j];
-      sQ[tid][j] = qq[j];
-    }
-    __syncthreads();
-    // channel c, nodes grp, grp+4, ...
-    const float udc = bf2f(th16[kOffUd + c]), uec = bf2f(th16[kOffUe + c]);
-    for (int ln = grp; ln < 256; ln += 4) {
-      const int64_t pp = t0 + ln;
-      if (pp >= E) break;
-      const float hp = bf2f(h[pp * kW + c]);
-      float asum = 0.f;
-      for (int j = 0; j < 4; ++j) {
-        const int q = sQ[ln][j];
-        if (q < 0) continue;
-        asum += sAg[ln][j];
-        pue += 0.5f * sAg[ln][j] * (hp + bf2f(h[(int64_t)q * kW + c]));
-      }
-      pud += sGn[ln] * hp;
-      dh[pp * kW + c] = sGn[ln] * udc + asum * uec;
-      if (c == 0) {
-        pcd += sGn[ln];
-        pce += 0.5f * asum;
-      }
-    }
-    __syncthreads();
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int sub = lane & 7, ch = 8 * sub, slot = lane >> 3;
+  float ud[8], ue[8], pud[8], pue[8];
+  float pcd = 0.f, pce = 0.f;
+#pragma unroll
+  for (int t = 0; t < 8; ++t) {
+    ud[t] = bf2f(th16[kOffUd + ch + t]);
+    ue[t] = bf2f(th16[kOffUe + ch + t]);
+    pud[t] = pue[t] = 0.f;
   }
-  // reduce the 4 groups in fixed order through LDS
-  __shared__ float red[4][2 * kW + 2];
-  red[grp][c] = pud;
-  red[grp][kW + c] = pue;
-  if (c == 0) {
-    red[grp][2 * kW] = pcd;
-    red[grp][2 * kW + 1] = pce;
+  for (int64_t p0 = (int64_t)blockIdx.x * 32; p0 < E; p0 += (int64_t)gridDim.x * 32) {
+    const int64_t p = p0 + wave * 8 + slot;
+    const bool on = p < E;
+    // lane sub < 4: neighbour sub; lane 4: the node's own coefficient; handed round below
+    int myq = -1;
+    float mine = 0.f;
+    if (on && sub < 4) {
+      myq = nbr[4 * p + sub];
+      if (myq >= 0)
+        mine = a[4 * p + sub] * float(gam_o[4 * p + sub] / sqrt(sdiag[p] * sdiag[myq]));
+    } else if (on && sub == 4) {
+      mine = float(gam_d[p] / sdiag[p]);
+    }
+    const float gn = __shfl(mine, 4, 8);
+    float hp[8];
+    h8u_t own = {0, 0, 0, 0};
+    if (on) own = *reinterpret_cast<const h8u_t*>(h + p * kW + ch);
+    h8u_t hq[4];
+    float ag[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int q = __shfl(myq, j, 8);
+      ag[j] = __shfl(mine, j, 8);
+      hq[j] = h8u_t{0, 0, 0, 0};
+      if (q >= 0) hq[j] = *reinterpret_cast<const h8u_t*>(h + (int64_t)q * kW + ch);
+    }
+    unpack8(own, hp);
+    float asum = 0.f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      float v[8];
+      unpack8(hq[j], v);
+      asum += ag[j];
+#pragma unroll
+      for (int t = 0; t < 8; ++t) pue[t] += 0.5f * ag[j] * (hp[t] + v[t]);
+    }
+    if (on) {
+      f4u_t lo, hi;
+#pragma unroll
+      for (int t = 0; t < 8; ++t) {
+        pud[t] += gn * hp[t];
+        (t < 4 ? lo : hi)[t & 3] = gn * ud[t] + asum * ue[t];
+      }
+      *reinterpret_cast<f4u_t*>(dh + p * kW + ch) = lo;
+      *reinterpret_cast<f4u_t*>(dh + p * kW + ch + 4) = hi;
+      pcd += gn;
+      pce += 0.5f * asum;
+    }
+  }
+  // the 8 node slots of a wave (fixed butterfly), then the 4 waves in order
+  __shared__ float red[4][kHeadPartial];
+#pragma unroll
+  for (int off = 8; off < 64; off <<= 1) {
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+      pud[t] += __shfl_xor(pud[t], off, 64);
+      pue[t] += __shfl_xor(pue[t], off, 64);
+    }
+    pcd += __shfl_xor(pcd, off, 64);
+    pce += __shfl_xor(pce, off, 64);
+  }
+  if (slot == 0) {
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+      red[wave][ch + t] = pud[t];
+      red[wave][kW + 1 + ch + t] = pue[t];
+    }
+    if (sub == 0) {
+      red[wave][kW] = pcd;
+      red[wave][2 * kW + 1] = pce;
+    }
   }
   __syncthreads();
-  for (int i = tid; i < kHeadPartial; i += 256)
-    partial[(int64_t)blockIdx.x * kHeadPartial + i] = red[0][i] + red[1][i] + red[2][i] + red[3][i];
+  if (tid < kHeadPartial)
+    partial[(int64_t)blockIdx.x * kHeadPartial + tid] = red[0][tid] + red[1][tid] + red[2][tid] + red[3][tid];
 }
 
-// Layer backward, part 1 (per tile of 64 nodes):
-//   dz = dh * (z > 0); partial dWh += h^T dz, dWm += m^T dz, db += dz;
-//   dh <- dh + dz Wh^T (in place); dm = dz Wm^T.
+// Layer backward, part 1 (per tile of 64 nodes, in = [h, m]):
+//   dz = dh * (z > 0); partial dW += in^T dz, db += dz; dh <- dh + dz Wh^T (in place);
+//   dm = dz Wm^T.
+// Both products run on the FP32 matrix cores (16 x 16 x 4 tiles, exact FP32 operands): wave w
+// owns the input channels 32w .. 32w + 31, its 32 weights per lane stay in registers over the
+// tiles. The node order of a dW step is b + 4 (lane >> 4) inside 16 nodes and the LDS strides
+// are 4 mod 64 floats, so that the operand reads of both products cover the 64 banks.
+// Bound by the matrix cores (256 products of 32 cycles per wave and tile, 3.4 us): 24,576
+// nodes took 122 us a layer with scalar products from LDS on 256 blocks, 26 us now.
+constexpr int kLdIn = kKA + 4;
+constexpr int kLdDz = kW + 4;
+
 __global__ __launch_bounds__(256) void k_layer_bwd(int E, const uint16_t* __restrict__ th16, int layer,
                                                    const uint16_t* __restrict__ h,
                                                    const uint16_t* __restrict__ m,
                                                    const float* __restrict__ z,
                                                    float* __restrict__ dh, float* __restrict__ dm,
                                                    float* __restrict__ partial) {
-  __shared__ float sIn[kTile][kKA + 1];
-  __shared__ float sDz[kTile][kW + 1];
-  __shared__ float sWt[kKA][kW + 1];  // W[k][c]
-  const int tid = threadIdx.x;
+  __shared__ alignas(16) float sIn[kTile][kLdIn];
+  __shared__ alignas(16) float sDz[kTile][kLdDz];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, lr = lane & 15, lq = lane >> 4;
   const int base = kLayerBase + layer * kLayerSize;
-  for (int i = tid; i < kKA * kW; i += 256) sWt[i / kW][i % kW] = bf2f(th16[base + i]);
-  const int c = tid & 63, g = tid >> 6;  // grad ownership: channel c, k in [32g, 32g+32)
-  float accW[32];
-  for (int i = 0; i < 32; ++i) accW[i] = 0.f;
+  // B operand of dz W^T: W[k][c] with k = 32 wave + 16 t + lr, c = 4 s + lq
+  float wreg[2][16];
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int s = 0; s < 16; ++s) wreg[t][s] = bf2f(th16[base + (32 * wave + 16 * t + lr) * kW + 4 * s + lq]);
+  float4_t accW[2][4];
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) accW[t][c] = float4_t{0.f, 0.f, 0.f, 0.f};
   float accB = 0.f;
   const int64_t n_tiles = (E + kTile - 1) / kTile;
-  for (int64_t t = blockIdx.x; t < n_tiles; t += gridDim.x) {
-    const int64_t p0 = t * kTile;
-    __syncthreads();
-    for (int i = tid; i < kTile * kW; i += 256) {
-      const int ln = i / kW, cc = i % kW;
+  for (int64_t tile = blockIdx.x; tile < n_tiles; tile += gridDim.x) {
+    const int64_t p0 = tile * kTile;
+    __syncthreads();  // the previous tile's operands are read
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int i = tid + 256 * u, ln = i >> 3, ch = 8 * (i & 7);
       const int64_t p = p0 + ln;
-      float hv = 0.f, mv = 0.f, dz = 0.f;
+      h8u_t hv = {0, 0, 0, 0}, mv = {0, 0, 0, 0};
       if (p < E) {
-        hv = bf2f(h[p * kW + cc]);
-        mv = bf2f(m[p * kW + cc]);
-        dz = z[p * kW + cc] > 0.f ? dh[p * kW + cc] : 0.f;
+        hv = *reinterpret_cast<const h8u_t*>(h + p * kW + ch);
+        mv = *reinterpret_cast<const h8u_t*>(m + p * kW + ch);
       }
-      sIn[ln][cc] = hv;
-      sIn[ln][kW + cc] = mv;
-      sDz[ln][cc] = dz;
+      float f[8], g[8];
+      unpack8(hv, f);
+      unpack8(mv, g);
+#pragma unroll
+      for (int t = 0; t < 8; ++t) {
+        sIn[ln][ch + t] = f[t];
+        sIn[ln][kW + ch + t] = g[t];
+      }
+    }
+    // dh in the layout of the second product's result (its accumulators start from it)
+    float4_t old[4][2];
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int64_t p = p0 + 16 * g + 4 * lq + i;
+          old[g][t][i] = (wave < 2 && p < E) ? dh[p * kW + 32 * wave + 16 * t + lr] : 0.f;
+        }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int i = tid + 256 * u, ln = i >> 4, ch = 4 * (i & 15);
+      const int64_t p = p0 + ln;
+      f4u_t zv = {0.f, 0.f, 0.f, 0.f}, dv = {0.f, 0.f, 0.f, 0.f};
+      if (p < E) {
+        zv = *reinterpret_cast<const f4u_t*>(z + p * kW + ch);
+        dv = *reinterpret_cast<const f4u_t*>(dh + p * kW + ch);
+      }
+#pragma unroll
+      for (int t = 0; t < 4; ++t) sDz[ln][ch + t] = zv[t] > 0.f ? dv[t] : 0.f;
     }
     __syncthreads();
-    for (int ln = 0; ln < kTile; ++ln) {
-      const float d = sDz[ln][c];
-      for (int i = 0; i < 32; ++i) accW[i] += sIn[ln][32 * g + i] * d;
-      if (g == 0) accB += d;
-    }
-    // d_in[ln][k] = sum_c dz[ln][c] W[k][c]; thread -> node ln = tid / 4, k chunk of 32
-    {
-      const int ln = tid >> 2, k0 = (tid & 3) * 32;
-      const int64_t p = p0 + ln;
-      float out[32];
-      for (int i = 0; i < 32; ++i) out[i] = 0.f;
-      for (int cc = 0; cc < kW; ++cc) {
-        const float d = sDz[ln][cc];
-        for (int i = 0; i < 32; ++i) out[i] += d * sWt[k0 + i][cc];
-      }
-      if (p < E) {
-        for (int i = 0; i < 32; ++i) {
-          const int k = k0 + i;
-          if (k < kW)
-            dh[p * kW + k] += out[i];
-          else
-            dm[p * kW + (k - kW)] = out[i];
+    // dW[k][c] += sum over nodes of in[node][k] dz[node][c]
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        const int node = 16 * g + b + 4 * lq;
+        const float a0 = sIn[node][32 * wave + lr], a1 = sIn[node][32 * wave + 16 + lr];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          const float d = sDz[node][16 * c + lr];
+          accW[0][c] = mfma_f32_4(a0, d, accW[0][c]);
+          accW[1][c] = mfma_f32_4(a1, d, accW[1][c]);
         }
       }
+    {
+      const int c = tid & 63, g = tid >> 6;
+#pragma unroll
+      for (int n = 0; n < 16; ++n) accB += sDz[16 * g + n][c];
+    }
+    // d_in[node][k] = sum_c dz[node][c] W[k][c], added to dh (k < 64) or stored as dm
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      float4_t o[2] = {old[g][0], old[g][1]};
+#pragma unroll
+      for (int s = 0; s < 16; ++s) {
+        const float d = sDz[16 * g + lr][4 * s + lq];
+        o[0] = mfma_f32_4(d, wreg[0][s], o[0]);
+        o[1] = mfma_f32_4(d, wreg[1][s], o[1]);
+      }
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int64_t p = p0 + 16 * g + 4 * lq + i;
+          const int k = 32 * wave + 16 * t + lr;
+          if (p >= E) continue;
+          if (wave < 2)
+            dh[p * kW + k] = o[t][i];
+          else
+            dm[p * kW + (k - kW)] = o[t][i];
+        }
     }
   }
   float* part = partial + (int64_t)blockIdx.x * kLayerPartial;
-  for (int i = 0; i < 32; ++i) part[(32 * g + i) * kW + c] = accW[i];
-  if (g == 0) part[2 * kW * kW + c] = accB;
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        part[(32 * wave + 16 * t + 4 * lq + i) * kW + 16 * c + lr] = accW[t][c][i];
+  __syncthreads();
+  sDz[wave][lane] = accB;
+  __syncthreads();
+  if (tid < kW) part[2 * kW * kW + tid] = sDz[0][tid] + sDz[1][tid] + sDz[2][tid] + sDz[3][tid];
 }
 
-// Layer backward, part 2: dh_p += sum_j a_pj dm_q (transpose of the message sum; a symmetric).
-__global__ void k_msg_bwd(int E, const int32_t* __restrict__ nbr, const float* __restrict__ a,
-                          const float* __restrict__ dm, float* __restrict__ dh) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (int64_t)E * kW) return;
-  const int64_t p = i / kW;
-  const int c = int(i % kW);
+// out[i] = sum_b partial[b][i], i < n: 64 columns a block, its 4 waves take the rows b = wave,
+// wave + 4, ... and are added in order.
+__device__ __forceinline__ void reduce_columns(int block, int nblocks, int stride, int n,
+                                               const float* __restrict__ partial, float* __restrict__ out,
+                                               float (*red)[64]) {
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int i = block * 64 + lane;
   float s = 0.f;
+  if (i < n) {
+#pragma unroll 16
+    for (int b = wave; b < nblocks; b += 4) s += partial[(int64_t)b * stride + i];
+  }
+  red[wave][lane] = s;
+  __syncthreads();
+  if (wave == 0 && i < n) out[i] = red[0][lane] + red[1][lane] + red[2][lane] + red[3][lane];
+}
+
+__global__ __launch_bounds__(256) void k_reduce_partials(int nblocks, int stride, int n,
+                                                         const float* __restrict__ partial,
+                                                         float* __restrict__ out) {
+  __shared__ float red[4][64];
+  reduce_columns(blockIdx.x, nblocks, stride, n, partial, out, red);
+}
+
+// Layer backward, part 2: dh_p += sum_j a_pj dm_q (transpose of the message sum; a symmetric),
+// 16 lanes a node. The first `red_blocks` blocks sum the layer's weight-gradient partials
+// instead: the two are independent, and a launch of its own for the sum (one thread per
+// weight walking 256 rows) took 53 us; both together take 8.0 us (the message sum alone took 11).
+__global__ __launch_bounds__(256) void k_msg_bwd(int E, const int32_t* __restrict__ nbr,
+                                                 const float* __restrict__ a, const float* __restrict__ dm,
+                                                 float* __restrict__ dh, int red_blocks, int nblocks, int stride,
+                                                 int n, const float* __restrict__ partial,
+                                                 float* __restrict__ out) {
+  __shared__ float red[4][64];
+  if ((int)blockIdx.x < red_blocks) {
+    reduce_columns(blockIdx.x, nblocks, stride, n, partial, out, red);
+    return;
+  }
+  const int64_t i = (int64_t)(blockIdx.x - red_blocks) * blockDim.x + threadIdx.x;
+  if (i >= (int64_t)E * (kW / 4)) return;
+  const int64_t p = i / (kW / 4);
+  const int c = 4 * int(i % (kW / 4));
+  f4u_t v[4];
+  float w[4];
+#pragma unroll
   for (int j = 0; j < 4; ++j) {
     const int q = nbr[4 * p + j];
-    if (q < 0) continue;
-    s += a[4 * p + j] * dm[(int64_t)q * kW + c];
+    w[j] = q >= 0 ? a[4 * p + j] : 0.f;
+    v[j] = f4u_t{0.f, 0.f, 0.f, 0.f};
+    if (q >= 0) v[j] = *reinterpret_cast<const f4u_t*>(dm + (int64_t)q * kW + c);
   }
-  dh[i] += s;
+  f4u_t o = *reinterpret_cast<const f4u_t*>(dh + p * kW + c);
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    float s = 0.f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) s += w[j] * v[j][t];
+    o[t] += s;
+  }
+  *reinterpret_cast<f4u_t*>(dh + p * kW + c) = o;
 }
 
-// Input layer backward: dz0 = dh * (z0 > 0); partial dW0 += x^T dz0, db0 += dz0.
+// Input layer backward: dz0 = dh * (z0 > 0); partial dW0 += x^T dz0, db0 += dz0. A wave takes
+// one node at a time (lane = channel), four nodes' loads issued together.
 __global__ __launch_bounds__(256) void k_input_bwd(int E, const float* __restrict__ x,
                                                    const float* __restrict__ z0,
                                                    const float* __restrict__ dh,
@@ -412,10 +578,24 @@ __global__ __launch_bounds__(256) void k_input_bwd(int E, const float* __restric
   const int tid = threadIdx.x, c = tid & 63, g = tid >> 6;
   float acc[kIn + 1];
   for (int i = 0; i <= kIn; ++i) acc[i] = 0.f;
-  for (int64_t p = (int64_t)blockIdx.x * 4 + g; p < E; p += (int64_t)gridDim.x * 4) {
-    const float d = z0[p * kW + c] > 0.f ? dh[p * kW + c] : 0.f;
-    for (int k = 0; k < kIn; ++k) acc[k] += x[p * kIn + k] * d;
-    acc[kIn] += d;
+  const int64_t step = (int64_t)gridDim.x * 4;
+  for (int64_t p0 = (int64_t)blockIdx.x * 4 + g; p0 < E; p0 += 4 * step) {
+    float d[4], zv[4], xv[4][kIn];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int64_t p = p0 + u * step < E ? p0 + u * step : p0;
+      zv[u] = z0[p * kW + c];
+      d[u] = dh[p * kW + c];
+#pragma unroll
+      for (int k = 0; k < kIn; ++k) xv[u][k] = x[p * kIn + k];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const float v = (p0 + u * step < E && zv[u] > 0.f) ? d[u] : 0.f;
+#pragma unroll
+      for (int k = 0; k < kIn; ++k) acc[k] += xv[u][k] * v;
+      acc[kIn] += v;
+    }
   }
   __shared__ float red[4][kIn + 1][kW];
   for (int k = 0; k <= kIn; ++k) red[g][k][c] = acc[k];
@@ -424,16 +604,6 @@ __global__ __launch_bounds__(256) void k_input_bwd(int E, const float* __restric
     const int k = i / kW, cc = i % kW;
     partial[(int64_t)blockIdx.x * kInPartial + i] = red[0][k][cc] + red[1][k][cc] + red[2][k][cc] + red[3][k][cc];
   }
-}
-
-// out[i] = sum_b partial[b][i] (fixed block order)
-__global__ void k_reduce_partials(int nblocks, int stride, int n, const float* __restrict__ partial,
-                                  float* __restrict__ out) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  float s = 0.f;
-  for (int b = 0; b < nblocks; ++b) s += partial[(int64_t)b * stride + i];
-  out[i] = s;
 }
 
 // ---------------------------------------------------------------------------
@@ -677,10 +847,6 @@ __global__ __launch_bounds__(256) void k_gemv(int n, const float* __restrict__ A
 constexpr int kInvN = 128;
 constexpr int kInvRS = 144;  // pivot-row LDS stride (16 mod 32 banks)
 constexpr int kInvCS = 18;   // pivot-column and per-wave scratch stride
-
-__device__ __forceinline__ float4_t mfma_f32_4(float a, float b, float4_t c) {
-  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
 
 __global__ __launch_bounds__(512) void k_spd_inverse_small(int n, float* __restrict__ A, int lda) {
   __shared__ float rowp[2][16][kInvRS];
@@ -1087,8 +1253,8 @@ int nfx_gnn_forward(int E, const int32_t* nbr, const float* a, const float* x, c
 
 int nfx_gnn_backward_workspace(int E) {
   (void)E;
-  // floats of the per-block partial buffer
-  return kBwdBlocks * kLayerPartial;
+  // floats of the per-block partial buffers: one layer's, the heads', the input layer's
+  return kBwdBlocks * kLayerPartial + kHeadBlocks * kHeadPartial + kInBlocks * kInPartial;
 }
 
 int nfx_gnn_backward(int E, const int32_t* nbr, const float* a, const float* x, const uint16_t* theta16,
@@ -1101,30 +1267,28 @@ int nfx_gnn_backward(int E, const int32_t* nbr, const float* a, const float* x, 
               "nfx_gnn_backward: null pointer");
   hipStream_t st = (hipStream_t)stream;
   const int64_t EW = (int64_t)E * kW;
-  hipLaunchKernelGGL(k_heads_bwd, dim3(kBwdBlocks), dim3(256), 0, st, E, nbr, a, theta16, h + kLayers * EW,
-                     sdiag, gamma_d, gamma_o, dh, partial);
+  float* part_heads = partial + kBwdBlocks * kLayerPartial;
+  float* part_in = part_heads + kHeadBlocks * kHeadPartial;
+  const int hb = std::min(grid_for(E, 32), kHeadBlocks), lb = std::min(grid_for(E, kTile), kBwdBlocks);
+  const int ib = std::min(grid_for(E, 16), kInBlocks);
+  const int red = grid_for(kLayerPartial, 64);
+  hipLaunchKernelGGL(k_heads_bwd, dim3(hb), dim3(256), 0, st, E, nbr, a, theta16, h + kLayers * EW, sdiag, gamma_d,
+                     gamma_o, dh, part_heads);
   NFX_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(256), 0, st, kBwdBlocks, kHeadPartial, kW, partial,
-                     grad + kOffUd);
-  hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(256), 0, st, kBwdBlocks, kHeadPartial, kW, partial + kW,
-                     grad + kOffUe);
-  hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(64), 0, st, kBwdBlocks, kHeadPartial, 1,
-                     partial + 2 * kW, grad + kOffCd);
-  hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(64), 0, st, kBwdBlocks, kHeadPartial, 1,
-                     partial + 2 * kW + 1, grad + kOffCe);
+  hipLaunchKernelGGL(k_reduce_partials, dim3(grid_for(kHeadPartial, 64)), dim3(256), 0, st, hb, kHeadPartial,
+                     kHeadPartial, part_heads, grad + kOffUd);
   NFX_LAUNCH_CHECK();
   for (int l = kLayers - 1; l >= 0; --l) {
-    hipLaunchKernelGGL(k_layer_bwd, dim3(kBwdBlocks), dim3(256), 0, st, E, theta16, l, h + l * EW, m + l * EW,
+    hipLaunchKernelGGL(k_layer_bwd, dim3(lb), dim3(256), 0, st, E, theta16, l, h + l * EW, m + l * EW,
                        z + (l + 1) * EW, dh, dm, partial);
     NFX_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_reduce_partials, dim3(grid_for(kLayerPartial, 256)), dim3(256), 0, st, kBwdBlocks,
+    hipLaunchKernelGGL(k_msg_bwd, dim3(red + grid_for(EW / 4, 256)), dim3(256), 0, st, E, nbr, a, dm, dh, red, lb,
                        kLayerPartial, kLayerPartial, partial, grad + kLayerBase + l * kLayerSize);
-    hipLaunchKernelGGL(k_msg_bwd, dim3(grid_for(EW, 256)), dim3(256), 0, st, E, nbr, a, dm, dh);
     NFX_LAUNCH_CHECK();
   }
-  hipLaunchKernelGGL(k_input_bwd, dim3(kBwdBlocks), dim3(256), 0, st, E, x, z, dh, partial);
-  hipLaunchKernelGGL(k_reduce_partials, dim3(grid_for(kInPartial, 256)), dim3(256), 0, st, kBwdBlocks,
-                     kInPartial, kInPartial, partial, grad + kOffW0);
+  hipLaunchKernelGGL(k_input_bwd, dim3(ib), dim3(256), 0, st, E, x, z, dh, part_in);
+  hipLaunchKernelGGL(k_reduce_partials, dim3(grid_for(kInPartial, 64)), dim3(256), 0, st, ib, kInPartial, kInPartial,
+                     part_in, grad + kOffW0);
   NFX_LAUNCH_CHECK();
   return NFX_OK;
 }
