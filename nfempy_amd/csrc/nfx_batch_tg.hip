@@ -14,6 +14,7 @@
 // The cycle z = x2 + W (r - S x2), x2 = x1 + P Ac^-1 P^T (r - S x1), x1 = W r is
 // symmetric; with the smoother a contraction in the S-norm it is SPD, as MINRES needs.
 #include "nfx_blockinv.h"
+#include "nfx_coarse_row.h"
 #include "nfx_common.h"
 
 namespace nfx {
@@ -255,34 +256,27 @@ __global__ __launch_bounds__(kTB) void k_btg_smoother(int n_cells, const double*
 }
 
 // Row a of the packed coarse operator of a's instance: sum over the cells p of a of the
-// entry sums of S_pp (column a) and of S_pk (column of the neighbour's aggregate).
-// One thread per aggregate, members in aggregate order: a fixed summation order.
+// entries of S_pp into a's own column and of S_pq into q's aggregate (FP64, one wave per row,
+// coarse_row_wave); the packed operators must be zero on entry.
 template <int NB>
-__global__ __launch_bounds__(64) void k_btg_coarse(int n_agg, const int32_t* __restrict__ agg_ptr,
-                                                   const int32_t* __restrict__ agg_mem,
-                                                   const int32_t* __restrict__ agg_of, const int32_t* __restrict__ nbr,
-                                                   const double* __restrict__ sd64, const double* __restrict__ so64,
-                                                   const int64_t* __restrict__ arow, const int32_t* __restrict__ a0,
-                                                   double* __restrict__ ac) {
-  const int ag = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ __launch_bounds__(256) void k_btg_coarse(int n_agg, const int32_t* __restrict__ agg_ptr,
+                                                    const int32_t* __restrict__ agg_mem,
+                                                    const int32_t* __restrict__ agg_of,
+                                                    const int32_t* __restrict__ nbr,
+                                                    const double* __restrict__ sd64, const double* __restrict__ so64,
+                                                    const int64_t* __restrict__ arow, const int32_t* __restrict__ a0,
+                                                    double* __restrict__ ac) {
+  const int ag = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
   if (ag >= n_agg) return;
-  double* row = ac + arow[ag];
-  const int base = a0[ag];
-  for (int k = agg_ptr[ag]; k < agg_ptr[ag + 1]; ++k) {
-    const int p = agg_mem[k];
-    double s = 0.0;
+  coarse_row_wave(ag, agg_ptr, agg_mem, agg_of, nbr,
+                  [&](int p, int s) {
+                    const double* b = s ? so64 + (4 * (int64_t)p + s - 1) * NB * NB : sd64 + (int64_t)p * NB * NB;
+                    double v = 0.0;
 #pragma unroll
-    for (int e = 0; e < NB * NB; ++e) s += sd64[(int64_t)p * NB * NB + e];
-    row[ag - base] += s;
-    for (int j = 0; j < 4; ++j) {
-      const int q = nbr[4 * p + j];
-      if (q < 0) continue;
-      double o = 0.0;
-#pragma unroll
-      for (int e = 0; e < NB * NB; ++e) o += so64[((int64_t)p * 4 + j) * NB * NB + e];
-      row[agg_of[q] - base] += o;
-    }
-  }
+                    for (int e = 0; e < NB * NB; ++e) v += b[e];
+                    return v;
+                  },
+                  ac + arow[ag], a0[ag]);
 }
 
 template <int NB>
@@ -666,10 +660,10 @@ int nfx_batch_tg_coarse(int nb, int n_agg, const int32_t* d_agg_ptr, const int32
               "nfx_batch_tg_coarse: null pointer");
   hipStream_t st = (hipStream_t)stream;
   if (nb == 1)
-    hipLaunchKernelGGL(k_btg_coarse<1>, dim3(grid_for(n_agg, 64)), dim3(64), 0, st, n_agg, d_agg_ptr, d_agg_mem,
+    hipLaunchKernelGGL(k_btg_coarse<1>, dim3(grid_for((int64_t)n_agg * 64, 256)), dim3(256), 0, st, n_agg, d_agg_ptr, d_agg_mem,
                        d_agg_of, d_nbr, d_sd64, d_so64, d_arow, d_a0, d_ac);
   else
-    hipLaunchKernelGGL(k_btg_coarse<4>, dim3(grid_for(n_agg, 64)), dim3(64), 0, st, n_agg, d_agg_ptr, d_agg_mem,
+    hipLaunchKernelGGL(k_btg_coarse<4>, dim3(grid_for((int64_t)n_agg * 64, 256)), dim3(256), 0, st, n_agg, d_agg_ptr, d_agg_mem,
                        d_agg_of, d_nbr, d_sd64, d_so64, d_arow, d_a0, d_ac);
   NFX_LAUNCH_CHECK();
   return NFX_OK;

@@ -15,6 +15,7 @@
 #include <algorithm>
 #include <vector>
 
+#include "nfx_coarse_row.h"
 #include "nfx_common.h"
 
 namespace nfx {
@@ -662,23 +663,19 @@ __global__ void k_agg_sum(int n_agg, int ns, int E, const int32_t* __restrict__ 
   C[i] = acc;
 }
 
-// Dense coarse operator row a: Ac[a][agg(q)] += S_pq for members p of a (FP64, member order).
-// Ac must be zero on entry.
-__global__ void k_coarse_dense(int n_agg, const int32_t* __restrict__ agg_ptr,
-                               const int32_t* __restrict__ agg_mem, const int32_t* __restrict__ agg_of,
-                               const int32_t* __restrict__ nbr, const double* __restrict__ sdiag,
-                               const double* __restrict__ soff, double* __restrict__ Ac) {
-  const int ag = blockIdx.x * blockDim.x + threadIdx.x;
+// Dense coarse operator row a: Ac[a][agg(q)] += S_pq for members p of a (FP64, one wave per
+// row, coarse_row_wave). Ac must be zero on entry.
+__global__ __launch_bounds__(256) void k_coarse_dense(int n_agg, const int32_t* __restrict__ agg_ptr,
+                                                      const int32_t* __restrict__ agg_mem,
+                                                      const int32_t* __restrict__ agg_of,
+                                                      const int32_t* __restrict__ nbr,
+                                                      const double* __restrict__ sdiag,
+                                                      const double* __restrict__ soff, double* __restrict__ Ac) {
+  const int ag = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
   if (ag >= n_agg) return;
-  double* row = Ac + (int64_t)ag * n_agg;
-  for (int k = agg_ptr[ag]; k < agg_ptr[ag + 1]; ++k) {
-    const int p = agg_mem[k];
-    row[ag] += sdiag[p];
-    for (int j = 0; j < 4; ++j) {
-      const int q = nbr[4 * p + j];
-      if (q >= 0) row[agg_of[q]] += soff[4 * p + j];
-    }
-  }
+  coarse_row_wave(ag, agg_ptr, agg_mem, agg_of, nbr,
+                  [&](int p, int s) { return s ? soff[4 * (int64_t)p + s - 1] : sdiag[p]; },
+                  Ac + (int64_t)ag * n_agg, 0);
 }
 
 // ---------------------------------------------------------------------------
@@ -739,23 +736,32 @@ __global__ void k_flux_bound_init(float* __restrict__ bound) {
 }
 
 // bound = max_i sum_j |M_ij| / M_ii over the flux-row ELL slots (the row-sum norm of
-// D^-1 M, an upper bound of its spectral radius); positive floats order as their bits
+// D^-1 M, an upper bound of its spectral radius); positive floats order as their bits. The
+// atomics on the one word are serial (one per wave took 84 us at 399,360 rows): a bounded grid
+// walks the rows, so at most kFluxBoundBlocks of them remain (84 -> 27 us).
+constexpr int kFluxBoundBlocks = 512;
+
 __global__ __launch_bounds__(256) void k_flux_bound(int n_u, int width, const int32_t* __restrict__ pos,
                                                     const int32_t* __restrict__ diag_pos,
                                                     const double* __restrict__ vals, float* __restrict__ bound) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  __shared__ float wmax[4];
   float b = 0.f;
-  if (i < n_u) {
+  for (int i = blockIdx.x * 256 + threadIdx.x; i < n_u; i += gridDim.x * 256) {
     double s = 0.0;
+#pragma unroll 4
     for (int k = 0; k < width; ++k) {
       const int q = pos[(int64_t)k * n_u + i];
       if (q >= 0) s += fabs(vals[q]);
     }
-    b = (float)(s / vals[diag_pos[i]]);
+    b = fmaxf(b, (float)(s / vals[diag_pos[i]]));
   }
   for (int off = 32; off > 0; off >>= 1) b = fmaxf(b, __shfl_xor(b, off, 64));
-  if ((threadIdx.x & 63) == 0 && b > 0.f)
-    atomicMax(reinterpret_cast<unsigned int*>(bound), __float_as_uint(b));
+  if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = b;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    b = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
+    if (b > 0.f) atomicMax(reinterpret_cast<unsigned int*>(bound), __float_as_uint(b));
+  }
 }
 
 // C = 2 omega D^-1 - omega^2 D^-1 M D^-1 on the flux-row ELL slots (FP64 arithmetic,
@@ -1198,8 +1204,8 @@ int nfx_flux_sweep_coef(int n_u, int width, const int32_t* pos, const int32_t* f
   hipStream_t st = (hipStream_t)stream;
   if (bound) {
     hipLaunchKernelGGL(k_flux_bound_init, dim3(1), dim3(64), 0, st, bound);
-    hipLaunchKernelGGL(k_flux_bound, dim3(grid_for(n_u, 256)), dim3(256), 0, st, n_u, width, pos, diag_pos, vals64,
-                       bound);
+    hipLaunchKernelGGL(k_flux_bound, dim3(std::min(grid_for(n_u, 256), kFluxBoundBlocks)), dim3(256), 0, st, n_u,
+                       width, pos, diag_pos, vals64, bound);
   }
   hipLaunchKernelGGL(k_flux_sweep_coef, dim3(grid_for((int64_t)width * n_u, 256)), dim3(256), 0, st, n_u, width,
                      pos, fcol, diag_pos, vals64, omega, bound, coef);
@@ -1331,7 +1337,7 @@ int nfx_coarse_dense(int n_agg, const int32_t* agg_ptr, const int32_t* agg_mem, 
   NFX_REQUIRE(n_agg >= 0, "nfx_coarse_dense: n_agg < 0");
   if (n_agg == 0) return NFX_OK;
   NFX_REQUIRE(agg_ptr && agg_mem && agg_of && nbr && sdiag && soff && Ac, "nfx_coarse_dense: null pointer");
-  hipLaunchKernelGGL(k_coarse_dense, dim3(grid_for(n_agg, 64)), dim3(64), 0, (hipStream_t)stream, n_agg,
+  hipLaunchKernelGGL(k_coarse_dense, dim3(grid_for((int64_t)n_agg * 64, 256)), dim3(256), 0, (hipStream_t)stream, n_agg,
                      agg_ptr, agg_mem, agg_of, nbr, sdiag, soff, Ac);
   NFX_LAUNCH_CHECK();
   return NFX_OK;

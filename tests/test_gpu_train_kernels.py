@@ -86,3 +86,54 @@ def test_network_backward_sizes(E):
         k = int(np.prod(shape))
         w, g = want[o:o + k], got[o:o + k]
         assert np.linalg.norm(g - w) <= 1e-4 * max(np.linalg.norm(w), 1e-3), (name, E)
+
+
+@pytest.mark.parametrize("sizes", [(1,), (12, 1, 51), (102, 103), (250, 7, 400), (3,) * 300])
+def test_coarse_operator_aggregate_sizes(sizes):
+    """P^T S P against numpy for aggregates of one cell, just below and above the cells a wave
+    holds at once (102), several batches, and many small ones; FP64 sums (1e-13 of the row)."""
+    import torch
+    from nfempy_amd import _native as nat
+
+    E, n_agg = sum(sizes), len(sizes)
+    nbr, sdiag, soff = _graph(E, n_agg)
+    rng = np.random.default_rng(E)
+    agg_of = rng.permutation(np.repeat(np.arange(n_agg), sizes))
+    mem = np.argsort(agg_of, kind="stable")
+    ptr = np.concatenate([[0], np.cumsum(sizes)])
+    i32, f64 = torch.int32, torch.float64
+    d = [_dev(a, i32) for a in (ptr, mem, agg_of, nbr)] + [_dev(sdiag, f64), _dev(soff, f64)]
+    Ac = torch.zeros((n_agg, n_agg), dtype=f64, device="cuda")
+    nat.call("nfx_coarse_dense", n_agg, *(nat.ptr(t) for t in d), nat.ptr(Ac), nat.stream_handle())
+    torch.cuda.synchronize()
+    want = np.zeros((n_agg, n_agg))
+    np.add.at(want, (agg_of, agg_of), sdiag)
+    p, j = np.nonzero(nbr >= 0)
+    np.add.at(want, (agg_of[p], agg_of[nbr[p, j]]), soff[p, j])
+    scale = np.abs(sdiag).sum()
+    assert np.abs(Ac.cpu().numpy() - want).max() <= 1e-13 * scale
+
+
+@pytest.mark.parametrize("n", [1, 255, 257, 150001])
+def test_flux_row_sum_bound(n):
+    """max_i sum_j |M_ij| / M_ii over tridiagonal rows (more rows than the kernel's grid covers in
+    one pass for the largest), a maximum: exact up to the FP32 rounding of each row's quotient."""
+    import torch
+    from nfempy_amd import _native as nat
+
+    rng = np.random.default_rng(n)
+    diag, off = rng.uniform(1.0, 2.0, n), rng.uniform(-0.4, 0.4, n)
+    vals = np.stack([diag, off, np.roll(off, 1)])  # slot-major; row i couples to i + 1 and i - 1
+    pos = np.arange(3 * n).reshape(3, n).copy()
+    pos[1, n - 1] = pos[2, 0] = -1
+    col = np.stack([np.arange(n), np.minimum(np.arange(n) + 1, n - 1), np.maximum(np.arange(n) - 1, 0)])
+    i32 = torch.int32
+    dpos, dcol, ddiag = _dev(pos, i32), _dev(col, i32), _dev(np.arange(n), i32)
+    dv = _dev(vals, torch.float64)
+    coef = torch.empty(3 * n, dtype=torch.float32, device="cuda")
+    bound = torch.full((1,), 7.0, dtype=torch.float32, device="cuda")
+    nat.call("nfx_flux_sweep_coef", n, 3, nat.ptr(dpos), nat.ptr(dcol), nat.ptr(ddiag), nat.ptr(dv), 0.0,
+             nat.ptr(coef), nat.ptr(bound), nat.stream_handle())
+    torch.cuda.synchronize()
+    s = diag + np.where(pos[1] >= 0, np.abs(vals[1]), 0) + np.where(pos[2] >= 0, np.abs(vals[2]), 0)
+    assert np.float32((s / diag).max()) == pytest.approx(bound.item(), rel=1.2e-7)
