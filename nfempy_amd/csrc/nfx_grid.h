@@ -1,0 +1,155 @@
+// Device-wide sums and vector exchange between the blocks of one cooperative launch.
+//
+// A Krylov iteration on a system of 1e3..1e5 rows is a handful of sums and short products; as launches
+// each costs 4-10 us whatever its work. A cooperative kernel keeps the blocks resident for the whole
+// solve, the operator and the vectors in LDS, and pays only for the exchange between blocks:
+//  * a sum: every block writes its partial into its slot (eight copies, so that readers spread over
+//    memory channels) and polls all slots of one copy. A slot is two 64-bit words, each half a double
+//    and the step's tag, so a reader needs no counter, no ordering between the words and no fence, and
+//    every block adds the same numbers in the same order;
+//  * a vector: stored and loaded with relaxed device-scope accesses (they pass the caches that are not
+//    coherent between XCDs); a block waits for its stores before it posts the next sum.
+// Device-scope fences instead of these accesses cost 5-30 us per step (measured, 8-256 blocks).
+// Two slot sets alternate: a block posts step k + 2 only after every block has read step k.
+//
+// Every wait is bounded (kGridWaitTicks): a block that gives up leaves, the others then give up in
+// their turn, the launch ends and the caller takes its general path.
+#pragma once
+
+#include "nfx_common.h"
+
+namespace nfx {
+
+// 1,024 against 512 threads, us an iteration of MINRES: 4.5 / 4.5 at 5,184 rows (30 k entries), 7.7 / 9.9 at
+// 41,088 rows (1.06 M entries) and 8.7 / 11.3 at 252,288 rows (1.9 M): more rows in flight beside the waits
+constexpr int kGridThreads = 1024;
+constexpr int kGridMaxBlocks = 256;
+constexpr int kGridCopies = 8;
+constexpr int64_t kGridSlotWords = 2 * (int64_t)kGridCopies * kGridMaxBlocks * 2;
+constexpr long long kGridWaitTicks = 50000000;  // 0.5 s of the 100 MHz clock
+constexpr int kGridLdsBytes = 158 * 1024;       // dynamic LDS of a block: all of a CU but the static arrays
+
+using grid_word = unsigned long long;
+
+template <typename T>
+__device__ __forceinline__ void grid_store(T* p, T v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename T>
+__device__ __forceinline__ T grid_load(const T* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Sums by cross-lane moves in the vector unit (a shuffle through the LDS unit takes ~50 ns a step, and
+// these steps are on the path of every iteration).
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_move(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWS, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
+
+// sum over the 64 lanes (all active), the same in every lane
+__device__ __forceinline__ double wave_total(double v) {
+  v += dpp_move<0x111, 0xf>(v);  // lane - 1, - 2, - 4, - 8 of the row of 16: its last lane has its sum
+  v += dpp_move<0x112, 0xf>(v);
+  v += dpp_move<0x114, 0xf>(v);
+  v += dpp_move<0x118, 0xf>(v);
+  v += dpp_move<0x142, 0xa>(v);  // last lane of rows 0, 2 into rows 1, 3
+  v += dpp_move<0x143, 0xc>(v);  // last lane of row 1 into rows 2, 3
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), 63),
+                          __builtin_amdgcn_readlane(__double2loint(v), 63));
+}
+
+template <int CTRL>
+__device__ __forceinline__ float dpp_move(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+
+// sum over groups of LANES (4, 8, 16) consecutive lanes, in every lane of the group
+template <int LANES>
+__device__ __forceinline__ float lanes_total(float v) {
+  v += dpp_move<0xb1>(v);  // neighbour, then neighbour pair
+  v += dpp_move<0x4e>(v);
+  if (LANES >= 8) v += dpp_move<0x141>(v);   // mirrored in 8: the other four
+  if (LANES >= 16) v += dpp_move<0x140>(v);  // mirrored in 16: the other eight
+  return v;
+}
+
+struct GridSync {
+  grid_word* slots;   // kGridSlotWords, zero before the launch
+  int nblk, rank;     // blocks that take part (at most kGridMaxBlocks and the threads of a block)
+  unsigned tag;       // steps posted so far
+  double (*post)[kGridThreads / 64];  // LDS, [2]
+  double (*part)[kGridThreads / 64];  // LDS, [2]
+  int (*good)[kGridThreads / 64];     // LDS, [2]
+};
+
+__device__ __forceinline__ grid_word* grid_slot(const GridSync& g, int copy, int b) {
+  return g.slots + (((int64_t)(g.tag & 1) * kGridCopies + copy) * kGridMaxBlocks + b) * 2;
+}
+
+// Adds the block's v (in wave order) and posts it. Contains a barrier; every exchange store that a
+// thread made before is complete when the post can be seen.
+__device__ __forceinline__ void grid_post(GridSync& g, double v) {
+  v = wave_total(v);
+  ++g.tag;
+  double* sh = g.post[g.tag & 1];
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (threadIdx.x < kGridCopies) {
+    double r = 0;
+#pragma unroll
+    for (int w = 0; w < kGridThreads / 64; ++w) r += sh[w];
+    const grid_word bits = (grid_word)__double_as_longlong(r);
+    grid_word* p = grid_slot(g, threadIdx.x, g.rank);
+    grid_store(p, (bits & 0xffffffff00000000ull) | g.tag);
+    grid_store(p + 1, (bits << 32) | g.tag);
+  }
+}
+
+// The sum of the last post over all blocks, the same in every thread. False: some wait was given up.
+// Contains a barrier.
+__device__ __forceinline__ bool grid_wait(GridSync& g, double& sum) {
+  const int waves = (g.nblk + 63) >> 6, wave = threadIdx.x >> 6;
+  if (wave < waves) {
+    double v = 0;
+    bool ok = true;
+    if ((int)threadIdx.x < g.nblk) {
+      const grid_word* p = grid_slot(g, g.rank % kGridCopies, threadIdx.x);
+      long long t0 = 0;
+      grid_word hi, lo;
+      for (int spin = 1;; ++spin) {
+        hi = grid_load(p);
+        lo = grid_load(p + 1);
+        if ((unsigned)hi == g.tag && (unsigned)lo == g.tag) break;
+        if ((spin & 63) == 0) {
+          const long long now = wall_clock64();
+          if (t0 == 0) t0 = now;
+          if (now - t0 > kGridWaitTicks) {
+            ok = false;
+            break;
+          }
+        }
+      }
+      v = __longlong_as_double((long long)((hi & 0xffffffff00000000ull) | (lo >> 32)));
+    }
+    v = wave_total(v);
+    ok = __all(ok);
+    if ((threadIdx.x & 63) == 0) {
+      g.part[g.tag & 1][wave] = v;
+      g.good[g.tag & 1][wave] = ok;
+    }
+  }
+  __syncthreads();
+  bool ok = true;
+  sum = 0;
+  for (int w = 0; w < waves; ++w) {
+    sum += g.part[g.tag & 1][w];
+    ok = ok && g.good[g.tag & 1][w];
+  }
+  return ok;
+}
+
+}  // namespace nfx

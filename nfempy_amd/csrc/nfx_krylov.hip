@@ -13,6 +13,7 @@
 
 #include "nfx_common.h"
 #include "nfx_el_twogrid.h"
+#include "nfx_minres_grid.h"
 #include "nfx_residual.h"
 
 namespace nfx {
@@ -24,17 +25,6 @@ constexpr int kMaxBlocks = 1024;
 // flight for the SpMV's gathers: the 32^3 x 6 Darcy solve (2,704 iterations) took 99 ms with
 // 256 threads, 75 ms with 512 in the A kernel and 72 ms in both; 1,024 threads took 105 ms.
 constexpr int kBlockMinres = 512;
-
-struct MinresState {
-  double beta, oldb, alfa, beta1;
-  double dbar, epsln, oldeps, phibar, cs, sn;
-  double delta, denom, phi;
-  double s, ratio;  // 1/beta and beta/oldb for the next A kernel
-  double rnorm2;    // scratch for norms
-  double bnorm2;
-  int stop;
-  int pad;
-};
 
 __device__ __forceinline__ double warp_sum(double v) {
   for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
@@ -172,55 +162,6 @@ __global__ __launch_bounds__(kBlock) void k_minres_init(int n, const float* __re
   }
   const double bs = block_sum(acc, sh);
   if (threadIdx.x == 0) partial_b[blockIdx.x] = bs;
-}
-
-// Scalar step of A(k): beta_k from B(k-1)'s partials, Givens rotation of
-// iteration k-1 (Paige-Saunders, as in SciPy's minres).
-__device__ __forceinline__ void minres_scalars(const MinresState& in, MinresState& out,
-                                               double beta, int first) {
-  out = in;
-  if (first) {
-    out.beta1 = beta;
-    out.beta = beta;
-    out.oldb = 0;
-    out.alfa = 0;
-    out.dbar = 0;
-    out.epsln = 0;
-    out.oldeps = 0;
-    out.phibar = beta;
-    out.cs = -1;
-    out.sn = 0;
-    out.delta = 0;
-    out.denom = 0;
-    out.phi = 0;
-    out.s = beta > 0 ? 1.0 / beta : 0.0;
-    out.ratio = 0;
-    out.stop = beta > 0 ? 0 : 1;
-    return;
-  }
-  const double alfa = in.alfa;
-  const double oldb = in.beta;
-  const double oldeps = in.epsln;
-  const double delta = in.cs * in.dbar + in.sn * alfa;
-  const double gbar = in.sn * in.dbar - in.cs * alfa;
-  const double epsln = in.sn * beta;
-  const double dbar = -in.cs * beta;
-  double gamma = hypot(gbar, beta);
-  if (gamma < 1e-300) gamma = 1e-300;
-  out.oldb = oldb;
-  out.beta = beta;
-  out.oldeps = oldeps;
-  out.delta = delta;
-  out.epsln = epsln;
-  out.dbar = dbar;
-  out.cs = gbar / gamma;
-  out.sn = beta / gamma;
-  out.phi = out.cs * in.phibar;
-  out.phibar = out.sn * in.phibar;
-  out.denom = 1.0 / gamma;
-  out.s = beta > 0 ? 1.0 / beta : 0.0;
-  out.ratio = oldb > 0 ? beta / oldb : 0.0;
-  if (!(beta > 0)) out.stop = 1;
 }
 
 // A(k): scalars, w/x update of iteration k-1 (unless first), then (unless
@@ -516,6 +457,8 @@ struct nfx_solver {
   int n = 0;
   int nnz = 0;
   hipStream_t stream = nullptr;
+  char* dev = nullptr;   // one device and one pinned allocation hold everything below
+  char* host = nullptr;
   float* buf = nullptr;  // 10 vectors of n floats
   double* r64 = nullptr;
   double* partial_a = nullptr;
@@ -523,6 +466,7 @@ struct nfx_solver {
   double* partial_r = nullptr;
   double* h_partial = nullptr;  // pinned
   MinresState* st = nullptr;    // 2 states
+  MinresGrid grid;
   // optional 3 x 3 block CSR copy of the FP32 operator (nfx_solver_set_block3)
   int b3_nbr = 0, b3_nblk = 0, blocks_a3 = 1;
   const int32_t* b3_rp = nullptr;
@@ -589,19 +533,39 @@ extern "C" int nfx_solver_create(nfx_solver** out, int n_rows, int nnz, void* st
   int bb = grid_for(n_rows, kBlockMinres);
   s->blocks_a = ba < kMaxBlocks ? ba : kMaxBlocks;
   s->blocks_b = bb < kMaxBlocks ? bb : kMaxBlocks;
-  hipError_t e = hipMalloc(&s->buf, sizeof(float) * (size_t)n_rows * 10);
-  if (e == hipSuccess) e = hipMalloc(&s->r64, sizeof(double) * (size_t)n_rows);
-  if (e == hipSuccess) e = hipMalloc(&s->partial_a, sizeof(double) * kMaxBlocks);
-  if (e == hipSuccess) e = hipMalloc(&s->partial_b, sizeof(double) * kMaxBlocks);
-  if (e == hipSuccess) e = hipMalloc(&s->partial_r, sizeof(double) * 2 * kResMaxBlocks);
-  if (e == hipSuccess) e = hipHostMalloc(&s->h_partial, sizeof(double) * 2 * kResMaxBlocks, hipHostMallocDefault);
-  if (e == hipSuccess) e = hipMalloc(&s->st, 2 * sizeof(MinresState));
-  if (e == hipSuccess) e = hipHostMalloc(&s->h_st, sizeof(MinresState), hipHostMallocDefault);
+  s->grid.max_blocks = minres_grid_capacity();
+  // pieces of one allocation each, at multiples of 256 bytes
+  size_t at = 0;
+  const auto piece = [&at](size_t bytes) {
+    const size_t here = at;
+    at += (bytes + 255) & ~(size_t)255;
+    return here;
+  };
+  const size_t o_buf = piece(sizeof(float) * (size_t)n_rows * 10), o_r64 = piece(sizeof(double) * (size_t)n_rows),
+               o_pa = piece(sizeof(double) * kMaxBlocks), o_pb = piece(sizeof(double) * kMaxBlocks),
+               o_pr = piece(sizeof(double) * 2 * kResMaxBlocks), o_st = piece(2 * sizeof(MinresState)),
+               o_slots = piece(sizeof(grid_word) * kGridSlotWords), o_res = piece(sizeof(GridResult));
+  hipError_t e = hipMalloc(&s->dev, at);
+  at = 0;
+  const size_t h_pr = piece(sizeof(double) * 2 * kResMaxBlocks), h_st = piece(sizeof(MinresState)),
+               h_res = piece(sizeof(GridResult));
+  if (e == hipSuccess) e = hipHostMalloc(&s->host, at, hipHostMallocDefault);
   if (e != hipSuccess) {
     set_error(std::string("nfx_solver_create: ") + hipGetErrorString(e));
     nfx_solver_destroy(s);
     return NFX_E_HIP;
   }
+  s->buf = reinterpret_cast<float*>(s->dev + o_buf);
+  s->r64 = reinterpret_cast<double*>(s->dev + o_r64);
+  s->partial_a = reinterpret_cast<double*>(s->dev + o_pa);
+  s->partial_b = reinterpret_cast<double*>(s->dev + o_pb);
+  s->partial_r = reinterpret_cast<double*>(s->dev + o_pr);
+  s->st = reinterpret_cast<MinresState*>(s->dev + o_st);
+  s->grid.slots = reinterpret_cast<grid_word*>(s->dev + o_slots);
+  s->grid.res = reinterpret_cast<GridResult*>(s->dev + o_res);
+  s->h_partial = reinterpret_cast<double*>(s->host + h_pr);
+  s->h_st = reinterpret_cast<MinresState*>(s->host + h_st);
+  s->grid.h_res = reinterpret_cast<GridResult*>(s->host + h_res);
   *out = s;
   return NFX_OK;
 }
@@ -628,14 +592,8 @@ extern "C" int nfx_solver_set_block3(nfx_solver* s, int n_blocks, const int32_t*
 
 extern "C" int nfx_solver_destroy(nfx_solver* s) {
   if (!s) return NFX_OK;
-  if (s->buf) (void)hipFree(s->buf);
-  if (s->r64) (void)hipFree(s->r64);
-  if (s->partial_a) (void)hipFree(s->partial_a);
-  if (s->partial_b) (void)hipFree(s->partial_b);
-  if (s->partial_r) (void)hipFree(s->partial_r);
-  if (s->h_partial) (void)hipHostFree(s->h_partial);
-  if (s->st) (void)hipFree(s->st);
-  if (s->h_st) (void)hipHostFree(s->h_st);
+  if (s->dev) (void)hipFree(s->dev);
+  if (s->host) (void)hipHostFree(s->host);
   delete s;
   return NFX_OK;
 }
@@ -764,6 +722,9 @@ extern "C" int nfx_solve_minres_ir(nfx_solver* s, const int32_t* d_rowptr, const
   int total = 0, outer = 0;
   double rel = 0;
   const int g = grid_for(n, kBlock);
+  // inner solves as one resident launch where the system fits the CUs' LDS, stepwise else and after
+  // a launch that could not do it (preconditioner not diagonal, blocks not resident in time)
+  int grid_blocks = s->b3_va ? 0 : minres_grid_blocks(&s->grid, n, s->nnz);
   for (; outer <= max_outer; ++outer) {
     double rr = 0, bb = 0;
     int rc = residual64(s, d_rowptr, d_col, d_val64, d_x, d_b, &rr, &bb);
@@ -775,9 +736,18 @@ extern "C" int nfx_solve_minres_ir(nfx_solver* s, const int32_t* d_rowptr, const
     hipLaunchKernelGGL(k_to_f32, dim3(g), dim3(kBlock), 0, s->stream, n, s->r64, d_sign, rn, rf);
     NFX_LAUNCH_CHECK();
     int it = 0;
-    rc = minres_inner(s, d_rowptr, d_col, d_val32, d_sign, d_pc_rowptr, d_pc_col, d_pc_val, rf, dx,
-                      inner_rtol, max_inner, &it);
-    if (rc) return rc;
+    if (grid_blocks) {
+      int status = 0;
+      rc = minres_grid_solve(&s->grid, grid_blocks, s->lanes, n, d_rowptr, d_col, d_val32, d_sign, d_pc_rowptr,
+                             d_pc_col, d_pc_val, rf, dx, s->buf, inner_rtol, max_inner, &it, &status, s->stream);
+      if (rc) return rc;
+      if (status) grid_blocks = 0;
+    }
+    if (!grid_blocks) {
+      rc = minres_inner(s, d_rowptr, d_col, d_val32, d_sign, d_pc_rowptr, d_pc_col, d_pc_val, rf, dx, inner_rtol,
+                        max_inner, &it);
+      if (rc) return rc;
+    }
     total += it;
     hipLaunchKernelGGL(k_axpy64, dim3(g), dim3(kBlock), 0, s->stream, n, rn, dx, d_x);
     NFX_LAUNCH_CHECK();

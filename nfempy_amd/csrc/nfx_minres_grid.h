@@ -1,0 +1,34 @@
+// Preconditioned FP32 MINRES of one system as one cooperative launch (nfx_minres_grid.hip).
+#pragma once
+
+#include "nfx_grid.h"
+#include "nfx_minres.h"
+
+namespace nfx {
+
+// what a launch reports
+struct GridResult {
+  int iters;
+  int status;  // 0 solved or out of iterations, 1 not applicable (nothing was done), 2 a wait was given up
+};
+
+// work space of a solver: the slots and the result
+struct MinresGrid {
+  int max_blocks = 0;  // 0: not available on this device
+  grid_word* slots = nullptr;
+  GridResult* res = nullptr;
+  GridResult* h_res = nullptr;  // pinned
+};
+
+int minres_grid_capacity();
+
+// Blocks for a system of n rows and nnz entries, 0 if it does not fit the blocks' LDS.
+int minres_grid_blocks(const MinresGrid* g, int n, int64_t nnz);
+
+// One inner solve with a diagonal preconditioner (CSR arrays as nfx_solve_minres_ir has them);
+// z: 2 n floats. *status as GridResult::status; *iters and x are set when it is 0.
+int minres_grid_solve(MinresGrid* g, int nblk, int lanes, int n, const int32_t* rp, const int32_t* ci, const float* va,
+                      const float* sign, const int32_t* prp, const int32_t* pci, const float* pva, const float* rhs,
+                      float* x, float* z, double tol, int maxit, int* iters, int* status, hipStream_t st);
+
+}  // namespace nfx
