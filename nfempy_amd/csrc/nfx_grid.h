@@ -25,7 +25,8 @@ namespace nfx {
 constexpr int kGridThreads = 1024;
 constexpr int kGridMaxBlocks = 256;
 constexpr int kGridCopies = 8;
-constexpr int64_t kGridSlotWords = 2 * (int64_t)kGridCopies * kGridMaxBlocks * 2;
+constexpr int kGridBlockWords = 2 * kGridCopies * 2;  // 64-bit words of slots per block
+constexpr int64_t kGridSlotWords = (int64_t)kGridBlockWords * kGridMaxBlocks;
 constexpr long long kGridWaitTicks = 50000000;  // 0.5 s of the 100 MHz clock
 constexpr int kGridLdsBytes = 158 * 1024;       // dynamic LDS of a block: all of a CU but the static arrays
 
@@ -77,7 +78,7 @@ __device__ __forceinline__ float lanes_total(float v) {
 }
 
 struct GridSync {
-  grid_word* slots;   // kGridSlotWords, zero before the launch
+  grid_word* slots;   // kGridBlockWords a block, zero before the launch
   int nblk, rank;     // blocks that take part (at most kGridMaxBlocks and the threads of a block)
   unsigned tag;       // steps posted so far
   double (*post)[kGridThreads / 64];  // LDS, [2]
@@ -86,7 +87,7 @@ struct GridSync {
 };
 
 __device__ __forceinline__ grid_word* grid_slot(const GridSync& g, int copy, int b) {
-  return g.slots + (((int64_t)(g.tag & 1) * kGridCopies + copy) * kGridMaxBlocks + b) * 2;
+  return g.slots + (((int64_t)(g.tag & 1) * kGridCopies + copy) * g.nblk + b) * 2;
 }
 
 // Adds the block's v (in wave order) and posts it. Contains a barrier; every exchange store that a
@@ -150,6 +151,72 @@ __device__ __forceinline__ bool grid_wait(GridSync& g, double& sum) {
     ok = ok && g.good[g.tag & 1][w];
   }
   return ok;
+}
+
+// what a launch (or one system of it) reports
+struct GridResult {
+  int iters;
+  int status;  // 0 solved or out of iterations, 1 not applicable (nothing was done), 2 a wait was given up
+};
+
+// The columns that a block's rows meet, as a list, and the rows' columns as 16-bit places in it.
+// Row i has entries start(i) .. start(i) + rowp[i + 1] - rowp[i] of ci; n columns in all.
+// bits, before: (n + 31) / 32 words each. grid_columns counts them (barriers inside; the count is the
+// same in every thread), grid_renumber writes list and idx.
+template <int LANES, typename Start>
+__device__ __forceinline__ int grid_columns(const int32_t* __restrict__ ci, int n, int R, const int* rowp, Start start,
+                                            unsigned* bits, int* before, int* scan) {
+  constexpr int T = kGridThreads;
+  const int t = threadIdx.x, nw = (n + 31) >> 5;
+  for (int w = t; w < nw; w += T) bits[w] = 0;
+  __syncthreads();
+  for (int i = t / LANES; i < R; i += T / LANES) {
+    const int32_t* c = ci + start(i);
+    for (int j = t % LANES, len = rowp[i + 1] - rowp[i]; j < len; j += LANES)
+      atomicOr(&bits[c[j] >> 5], 1u << (c[j] & 31));
+  }
+  __syncthreads();
+  // exclusive prefix of the bit counts: a run of words per thread, then waves, then the block
+  const int run = (nw + T - 1) / T, w0 = min(nw, t * run), w1 = min(nw, w0 + run);
+  int cnt = 0;
+  for (int w = w0; w < w1; ++w) cnt += __popc(bits[w]);
+  int inc = cnt;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int o = __shfl_up(inc, off, 64);
+    if ((t & 63) >= off) inc += o;
+  }
+  if ((t & 63) == 63) scan[t >> 6] = inc;
+  __syncthreads();
+  int pre = inc - cnt, total = 0;
+  for (int w = 0; w < T / 64; ++w) {
+    if (w < (t >> 6)) pre += scan[w];
+    total += scan[w];
+  }
+  for (int w = w0; w < w1; ++w) {
+    before[w] = pre;
+    pre += __popc(bits[w]);
+  }
+  __syncthreads();
+  return total;
+}
+
+template <int LANES, typename Start>
+__device__ __forceinline__ void grid_renumber(const int32_t* __restrict__ ci, int n, int R, const int* rowp,
+                                              Start start, const unsigned* bits, const int* before, int* list,
+                                              unsigned short* idx) {
+  constexpr int T = kGridThreads;
+  const int t = threadIdx.x, nw = (n + 31) >> 5;
+  for (int w = t; w < nw; w += T) {
+    int p = before[w];
+    for (unsigned b = bits[w]; b; b &= b - 1) list[p++] = 32 * w + __ffs(b) - 1;
+  }
+  for (int i = t / LANES; i < R; i += T / LANES) {
+    const int32_t* c = ci + start(i);
+    for (int j = t % LANES, len = rowp[i + 1] - rowp[i]; j < len; j += LANES)
+      idx[rowp[i] + j] = (unsigned short)(before[c[j] >> 5] + __popc(bits[c[j] >> 5] & ((1u << (c[j] & 31)) - 1)));
+  }
+  __syncthreads();
 }
 
 }  // namespace nfx

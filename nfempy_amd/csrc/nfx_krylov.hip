@@ -11,6 +11,7 @@
 #include <cmath>
 #include <vector>
 
+#include "nfx_bm_grid.h"
 #include "nfx_common.h"
 #include "nfx_el_twogrid.h"
 #include "nfx_minres_grid.h"
@@ -1190,7 +1191,7 @@ struct nfx_minres_batch {
   std::vector<int32_t> h_tile_ptr;
   int n_act = 0;
   int32_t* mode = nullptr;
-  float* buf = nullptr;  // 10 vectors of n_total floats
+  float* buf = nullptr;  // 13 vectors of n_total floats
   double* r64 = nullptr;
   double* pa = nullptr;  // n_tiles partials (alpha / r.r)
   double* pb = nullptr;  // n_tiles partials (y'.z / b.b)
@@ -1201,6 +1202,7 @@ struct nfx_minres_batch {
   int32_t* h_mode = nullptr;
   double* h_sums = nullptr;
   double* h_scale = nullptr;
+  nfx::BmGrid grid;
   std::vector<nfx_batch_tg> pc;  // two-grid groups on the pressure rows (optional)
 };
 
@@ -1223,6 +1225,7 @@ static void bm_free(nfx_minres_batch* s) {
   (void)hipHostFree(s->h_mode);
   (void)hipHostFree(s->h_sums);
   (void)hipHostFree(s->h_scale);
+  nfx::bm_grid_destroy(&s->grid);
   delete s;
 }
 
@@ -1260,7 +1263,7 @@ extern "C" int nfx_minres_batch_create(nfx_minres_batch** out, int n_inst, const
   if (e == hipSuccess) e = hipMalloc(&s->mode, sizeof(int32_t) * n_inst);
   if (e == hipSuccess) e = hipMalloc(&s->act, sizeof(int32_t) * s->n_tiles);
   if (e == hipSuccess) e = hipHostMalloc(&s->h_act, sizeof(int32_t) * s->n_tiles, hipHostMallocDefault);
-  if (e == hipSuccess) e = hipMalloc(&s->buf, sizeof(float) * (size_t)off * 10);
+  if (e == hipSuccess) e = hipMalloc(&s->buf, sizeof(float) * (size_t)off * 13);
   if (e == hipSuccess) e = hipMalloc(&s->r64, sizeof(double) * (size_t)off);
   if (e == hipSuccess) e = hipMalloc(&s->pa, sizeof(double) * s->n_tiles);
   if (e == hipSuccess) e = hipMalloc(&s->pb, sizeof(double) * s->n_tiles);
@@ -1282,6 +1285,11 @@ extern "C" int nfx_minres_batch_create(nfx_minres_batch** out, int n_inst, const
     return NFX_E_HIP;
   }
   s->h_tile_ptr = tile_ptr;
+  const int rc = nfx::bm_grid_create(&s->grid, n_inst, items.data(), s->items, s->stream);
+  if (rc) {
+    bm_free(s);
+    return rc;
+  }
   *out = s;
   return NFX_OK;
 }
@@ -1485,10 +1493,24 @@ extern "C" int nfx_solve_minres_batch_ir(nfx_minres_batch* s, const double* d_b,
     NFX_LAUNCH_CHECK();
     // the inner solve changes h_mode: keep the outer set for the update that follows
     std::vector<int32_t> mode_outer(s->h_mode, s->h_mode + m);
-    rc = bm_inner(s, rf, dx, tol.data(), max_inner, it.data());
+    // instances that fit a few CUs as resident launches, the rest stepwise together
+    std::vector<char> done;
+    std::vector<int> resident(m, 0);
+    rc = nfx::bm_grid_solve(&s->grid, m, N, s->items, s->mode, s->h_mode, s->pc, rf, dx, s->buf, s->buf + N * 10, tol.data(),
+                            max_inner, resident.data(), &done, st);
     if (rc) return rc;
+    bool rest = false;
     for (int i = 0; i < m; ++i) {
-      h_iters[i] += it[i];
+      if (done[i]) s->h_mode[i] = 2;
+      rest = rest || s->h_mode[i] == 0;
+    }
+    std::fill(it.begin(), it.end(), 0);
+    if (rest) {
+      rc = bm_inner(s, rf, dx, tol.data(), max_inner, it.data());
+      if (rc) return rc;
+    }
+    for (int i = 0; i < m; ++i) {
+      h_iters[i] += done[i] ? resident[i] : it[i];
       s->h_mode[i] = mode_outer[i];
     }
     NFX_CHECK_HIP(hipMemcpyAsync(s->mode, s->h_mode, sizeof(int32_t) * m, hipMemcpyHostToDevice, st));

@@ -6,12 +6,6 @@
 
 namespace nfx {
 
-// what a launch reports
-struct GridResult {
-  int iters;
-  int status;  // 0 solved or out of iterations, 1 not applicable (nothing was done), 2 a wait was given up
-};
-
 // work space of a solver: the slots and the result
 struct MinresGrid {
   int max_blocks = 0;  // 0: not available on this device

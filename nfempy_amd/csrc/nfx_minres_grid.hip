@@ -86,50 +86,16 @@ __global__ __launch_bounds__(kGridThreads) void k_minres_grid(MinresGridArgs a) 
   if (fits) {
     unsigned* bits = reinterpret_cast<unsigned*>(lds + base);
     int* before = reinterpret_cast<int*>(bits + nw);
-    for (int w = t; w < nw; w += T) bits[w] = 0;
+    for (int i = t; i <= R; i += T) rowp[i] = a.rp[r0 + i] - e0;
     __syncthreads();
-    for (int j = t; j < nz; j += T) {
-      const int c = a.ci[e0 + j];
-      atomicOr(&bits[c >> 5], 1u << (c & 31));
-    }
-    __syncthreads();
-    // exclusive prefix of the bit counts: a run of words per thread, then waves, then the block
-    const int run = (nw + T - 1) / T, w0 = min(nw, t * run), w1 = min(nw, w0 + run);
-    int cnt = 0;
-    for (int w = w0; w < w1; ++w) cnt += __popc(bits[w]);
-    int inc = cnt;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const int o = __shfl_up(inc, off, 64);
-      if ((t & 63) >= off) inc += o;
-    }
-    if ((t & 63) == 63) sh_scan[t >> 6] = inc;
-    __syncthreads();
-    int pre = inc - cnt;
-    for (int w = 0; w < T / 64; ++w) {
-      if (w < (t >> 6)) pre += sh_scan[w];
-      H += sh_scan[w];
-    }
-    for (int w = w0; w < w1; ++w) {
-      before[w] = pre;
-      pre += __popc(bits[w]);
-    }
+    const auto start = [&](int i) { return e0 + rowp[i]; };
+    H = grid_columns<LANES>(a.ci, n, R, rowp, start, bits, before, sh_scan);
     // room for the list above the bits, and for vectors + z below it
     fits = H <= 65535 && base + 8 * (int64_t)nw + 4 * (int64_t)H <= a.lds &&
            base + 4 * (9 * (int64_t)R + 2 * (int64_t)H) <= a.lds;
     if (fits) {
       list = reinterpret_cast<int*>(lds + a.lds) - H;
-      __syncthreads();
-      for (int w = t; w < nw; w += T) {
-        int p = before[w];
-        for (unsigned b = bits[w]; b; b &= b - 1) list[p++] = 32 * w + __ffs(b) - 1;
-      }
-      for (int i = t; i <= R; i += T) rowp[i] = a.rp[r0 + i] - e0;
-      for (int j = t; j < nz; j += T) {
-        const int c = a.ci[e0 + j];
-        idx[j] = (unsigned short)(before[c >> 5] + __popc(bits[c >> 5] & ((1u << (c & 31)) - 1)));
-      }
-      __syncthreads();
+      grid_renumber<LANES>(a.ci, n, R, rowp, start, bits, before, list, idx);
       const int lane = t % LANES;
       for (int i = t / LANES; i < R; i += T / LANES) {
         const float sg = a.sign ? a.sign[r0 + i] : 1.f;

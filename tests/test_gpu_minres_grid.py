@@ -110,3 +110,30 @@ def test_exact_breakdown_is_finite():
     x, info = s.solve(b, rtol=1e-12)
     assert info["converged"] and float((x - b).norm() / b.norm()) <= 1e-12
     s.close()
+
+
+@pytest.mark.parametrize("pc", ["diag", "twogrid", "learned"])
+def test_batch_over_resident_sizes(pc):
+    """Instances of one block, of many, more blocks than fit one launch, and (11 cubed: 216 aggregates)
+    one that the two-grid cycle leaves to the stepwise kernels: FP64 residuals, and each instance bitwise
+    what it is alone (its block count follows from its own size)."""
+    import torch
+
+    from nfempy_amd.batch import DarcyBatch
+
+    specs = [(2, 1), (9, 2), (11, 1), (5, 2), (9, 2), (7, 1), (1, 2), (9, 2)]
+    b = DarcyBatch(specs, seed=4, workers=1)
+    b.assemble()
+    print(f"[minres grid] batch {pc}", flush=True)
+    xs, infos, _ = b.solve_batched(rtol=1e-8, pc=pc)
+    for i in range(len(specs)):
+        assert infos[i]["converged"], (i, infos[i])
+        y = b.fp64_system(i)
+        n = len(y["rowptr"]) - 1
+        A = torch.sparse_csr_tensor(y["rowptr"].long(), y["col"].long(), y["vals64"], size=(n, n))
+        res = float((y["b"] - A @ xs[i]).norm() / y["b"].norm())
+        assert res <= 1.1e-8, (i, res)
+    for i in (1, 2, 3, 6):
+        alone, info, _ = b.solve_batched([i], rtol=1e-8, pc=pc)
+        assert info[0]["iterations"] == infos[i]["iterations"]
+        assert torch.equal(alone[0], xs[i]), i
