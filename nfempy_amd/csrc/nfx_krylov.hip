@@ -13,6 +13,7 @@
 
 #include "nfx_bm_grid.h"
 #include "nfx_common.h"
+#include "nfx_el_grid.h"
 #include "nfx_el_twogrid.h"
 #include "nfx_minres_grid.h"
 #include "nfx_residual.h"
@@ -848,6 +849,8 @@ extern "C" int nfx_solve_minres_ir_tg(nfx_solver* s, const int32_t* d_rowptr, co
   int total = 0, outer = 0;
   double rel = 0;
   const int g = grid_for(n, kBlock);
+  // as one resident launch where the block operator and the preconditioner fit the CUs' LDS
+  int grid_blocks = s->b3_va ? el_grid_blocks(el_grid_capacity(), pc, s->b3_nblk) : 0;
   for (; outer <= max_outer; ++outer) {
     double rr = 0, bb = 0;
     int rc = residual64(s, d_rowptr, d_col, d_val64, d_x, d_b, &rr, &bb);
@@ -859,8 +862,17 @@ extern "C" int nfx_solve_minres_ir_tg(nfx_solver* s, const int32_t* d_rowptr, co
     hipLaunchKernelGGL(k_to_f32, dim3(g), dim3(kBlock), 0, s->stream, n, s->r64, nullptr, rn, rf);
     NFX_LAUNCH_CHECK();
     int it = 0;
-    rc = minres_inner_tg(s, d_rowptr, d_col, d_val32, pc, rf, dx, inner_rtol, max_inner, &it);
-    if (rc) return rc;
+    if (grid_blocks) {
+      int status = 0;
+      rc = el_grid_solve(&s->grid, grid_blocks, n, s->b3_nblk, s->b3_rp, s->b3_ci, s->b3_va, pc, rf, dx, s->buf,
+                         inner_rtol, max_inner, &it, &status, s->stream);
+      if (rc) return rc;
+      if (status) grid_blocks = 0;
+    }
+    if (!grid_blocks) {
+      rc = minres_inner_tg(s, d_rowptr, d_col, d_val32, pc, rf, dx, inner_rtol, max_inner, &it);
+      if (rc) return rc;
+    }
     total += it;
     hipLaunchKernelGGL(k_axpy64, dim3(g), dim3(kBlock), 0, s->stream, n, rn, dx, d_x);
     NFX_LAUNCH_CHECK();

@@ -137,3 +137,41 @@ def test_batch_over_resident_sizes(pc):
         alone, info, _ = b.solve_batched([i], rtol=1e-8, pc=pc)
         assert info[0]["iterations"] == infos[i]["iterations"]
         assert torch.equal(alone[0], xs[i]), i
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 5, 9])
+def test_elasticity_resident_matches_stepwise(n):
+    """The resident solve takes the 3 x 3 block operator; without it the stepwise kernels run. Both end at
+    an FP64 residual of 1e-9; the system's conditioning separates their solutions by more."""
+    import torch
+
+    from nfempy_amd.elasticity import ElasticitySystem
+    from nfempy_amd.mesh import Mesh, unit_cube
+    from nfempy_amd.spaces import ProductSpace
+
+    mesh = Mesh.from_blocks(3, *unit_cube(n))
+    space = ProductSpace({"s": (3, 3, "BDM", 1, mesh), "u": (3, 3, "Lagrange", 0, mesh),
+                          "t": (3, 3, "Lagrange", 0, mesh)})
+    space.make_subspaces_discontinuous({"u": True, "t": True})
+    space.build_structures({"s": [1], "u": [1], "t": [1]}, {"s": [2, 3, 4, 5, 6, 7]})
+    r = np.random.default_rng(n)
+    lam, mu = (np.exp(0.5 * r.standard_normal(6 * n ** 3)) for _ in range(2))
+    rhs = lambda x, y, z: np.array([0.3 * np.ones_like(x), 0.7 * np.ones_like(x), np.ones_like(x)]
+                                   + [np.zeros_like(x)] * 3)
+    y = ElasticitySystem(space, {"lambda": lam, "mu": mu, "rhs": rhs})
+    for fp64 in (True, False):
+        y.assemble("A", fp64=fp64)
+    got = {}
+    for block3 in (True, False):
+        y.use_block3 = block3
+        print(f"[minres grid] elasticity n={n} blocks={block3}", flush=True)
+        x, info = y.solve(rtol=1e-9)
+        assert info["converged"] and info["residual"] <= 1e-9, info
+        rp, col, _, v64 = y.full("A")
+        A = torch.sparse_csr_tensor(rp.long(), col.long(), v64, size=(y.n, y.n))
+        res = float((-y.rhs64 - A @ x).norm() / y.rhs64.norm())
+        assert res <= 1.1e-9, res
+        got[block3] = x, info["iterations"]
+    assert abs(got[True][1] - got[False][1]) <= 48
+    err = float((got[True][0] - got[False][0]).norm() / got[False][0].norm())
+    assert err <= 1e-6, err
