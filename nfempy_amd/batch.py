@@ -224,7 +224,9 @@ class DarcyBatch:
         for d, g in self.groups.items():
             if only is not None and d != only:
                 continue
-            grid = g["grid"] or min(g["n_tiles"], 2048)
+            # a tile a block up to 4,096: 2,480 tiles of RT2 took 22.8 us on 2,048 blocks, 21.0 on as many
+            # as tiles (a block's second tile waits for its first)
+            grid = g["grid"] or min(g["n_tiles"], 4096)
             nat.call("nfx_assemble_darcy_batched", len(self.instances), nat.ptr(self._items), g["n_tiles"],
                      nat.ptr(g["tiles"]), g["tile_rows"], max(grid, 1), d, nat.stream_handle(stream))
 

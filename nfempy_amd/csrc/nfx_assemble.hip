@@ -461,19 +461,6 @@ __device__ __forceinline__ void darcy_row_tile(
   const int rl = min(r0 + n_in_tile, n_rows);
   const bool per_element = (ks_q == 0 && fs_q == 0);
   if (RS_ONLY && !per_element) return;
-  // the reference-tensor path reads only Rs | Bc | ck; a caller that already holds the
-  // table in st (same element, same path) passes load_table = false
-  if (load_table) {
-    if constexpr (RS_ONLY) {
-      for (int i = threadIdx.x; i < NT - NT_RS; i += TILE) st[i] = tab[NT_RS + i];
-    } else {
-      for (int i = (per_element ? NT_RS : 0) + threadIdx.x; i < NT; i += TILE) st[i] = tab[i];
-    }
-  }
-  const int base = rowptr[r0];
-  const int span = rowptr[rl] - base;
-  for (int i = threadIdx.x; i < span; i += TILE) sv[i] = R(0);
-  __syncthreads();
   const R* tw = st;
   const R* tphi = st + NQ;
   const R* tdiv = tphi + NQ * NB * DIM;
@@ -482,6 +469,12 @@ __device__ __forceinline__ void darcy_row_tile(
   const R* tBc = tRs + NB * NB * NS;
   const R* tck = tBc + NB * NP;
   RowLoad<DIM, R, GEO> in[RPT];
+  // column positions of the longer rows, five words an incidence: with the incidences, ahead of the
+  // loads that depend on those (RS_ONLY: registers are left for them)
+  constexpr bool POS_EARLY = RS_ONLY && RPT == 1 && !row_pos_packed(NL) && row_pos_stride(NL) % 4 == 0;
+  constexpr int NPW = POS_EARLY ? row_pos_stride(NL) / 4 : 1;
+  uint32_t pwd[2][NPW];
+  int off_early = 0;
   // load phase: incidences, then signs / metric (or vertices) / coefficients
 #pragma unroll
   for (int h = 0; h < RPT; ++h) {
@@ -495,6 +488,15 @@ __device__ __forceinline__ void darcy_row_tile(
       if constexpr (row_pos_packed(NL))
         in[h].pw[j] = (OFF_PACKED ? r < rl : c >= 0) ? reinterpret_cast<const uint32_t*>(pos)[(int64_t)r * 2 + j] : 0u;
     }
+  }
+  if constexpr (POS_EARLY) {
+    const int r = r0 + threadIdx.x;
+    const uint32_t* pw = reinterpret_cast<const uint32_t*>(pos) + (int64_t)(r < rl ? r : r0) * 2 * NPW;
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int w = 0; w < NPW; ++w) pwd[j][w] = pw[j * NPW + w];
+    off_early = rowptr[r < rl ? r : r0];
   }
 #pragma unroll
   for (int h = 0; h < RPT; ++h) {
@@ -542,6 +544,21 @@ __device__ __forceinline__ void darcy_row_tile(
       }
     }
   }
+  // The table and the row starts come beside the loads above, not before them (41,154 RT2 tetrahedra
+  // 33.6 -> 31.3 us, a 4 x 4 x 4 mesh of RT1 6.5 -> 6.2 us).
+  // the reference-tensor path reads only Rs | Bc | ck; a caller that already holds the
+  // table in st (same element, same path) passes load_table = false
+  if (load_table) {
+    if constexpr (RS_ONLY) {
+      for (int i = threadIdx.x; i < NT - NT_RS; i += TILE) st[i] = tab[NT_RS + i];
+    } else {
+      for (int i = (per_element ? NT_RS : 0) + threadIdx.x; i < NT; i += TILE) st[i] = tab[i];
+    }
+  }
+  const int base = rowptr[r0];
+  const int span = rowptr[rl] - base;
+  for (int i = threadIdx.x; i < span; i += TILE) sv[i] = R(0);
+  __syncthreads();
   // compute phase
 #pragma unroll
   for (int h = 0; h < RPT; ++h) {
@@ -552,6 +569,8 @@ __device__ __forceinline__ void darcy_row_tile(
     if constexpr (OFF_PACKED) {
       static_assert(row_off_packed(NL) && TILE == 128 && RPT == 1, "packed offsets: 128-row tiles");
       off = (int)((L.pw[0] >> 25) | ((L.pw[1] >> 25) << 7));
+    } else if constexpr (POS_EARLY) {
+      off = off_early - base;
     } else {
       off = rowptr[r] - base;
     }
@@ -647,7 +666,7 @@ __device__ __forceinline__ void darcy_row_tile(
         const uint32_t* pw = reinterpret_cast<const uint32_t*>(pos) + ((int64_t)r * 2 + j) * NW;
         uint32_t wd[NW];
 #pragma unroll
-        for (int w = 0; w < NW; ++w) wd[w] = pw[w];
+        for (int w = 0; w < NW; ++w) wd[w] = POS_EARLY ? pwd[j][POS_EARLY ? w : 0] : pw[w];
 #pragma unroll
         for (int b = 0; b < NL; ++b) {
           const int p = (wd[b >> 2] >> (8 * (b & 3))) & 0xff;
@@ -700,7 +719,7 @@ constexpr int row_kernel_min_waves() {
   return (NB <= 4 && sizeof(R) == 4) ? 8 : 1;
 }
 
-template <int DIM, int NB, int NP, int NQ, typename R, bool GEO>
+template <int DIM, int NB, int NP, int NQ, typename R, bool GEO, bool RS_ONLY = false>
 __global__ __launch_bounds__(kRowsPerBlock)
 __attribute__((amdgpu_waves_per_eu(row_kernel_min_waves<NB, R>(), 8))) void k_darcy_rows(
     int n_rows, const int32_t* __restrict__ inc, const uint8_t* __restrict__ pos,
@@ -710,7 +729,7 @@ __attribute__((amdgpu_waves_per_eu(row_kernel_min_waves<NB, R>(), 8))) void k_da
     R* __restrict__ vals, R* __restrict__ rhs, DarcyRowBc<R> bc, const R* __restrict__ geo,
     const int32_t* __restrict__ tile_map, int n_map) {
   constexpr int NL = NB + NP;
-  constexpr int NT = DarcyTab<DIM, NB, NP, NQ>::NT;
+  constexpr int NT = DarcyTab<DIM, NB, NP, NQ>::NT - (RS_ONLY ? NQ * (1 + NB * DIM + NB + NP) : 0);
   constexpr int RPT = row_kernel_rpt<NB, R>();
   __shared__ R st[NT];
   __shared__ R sv[kRowsPerBlock * RPT * 2 * NL];
@@ -733,7 +752,7 @@ __attribute__((amdgpu_waves_per_eu(row_kernel_min_waves<NB, R>(), 8))) void k_da
     for (int i = blockIdx.x; i < n_slots; i += gridDim.x) {
       const int t = tile_map ? tile_map[i] : i;
       if (t < 0 || t >= n_tiles) continue;
-      darcy_row_tile<DIM, NB, NP, NQ, kRowsPerBlock, R, GEO, RPT>(t * kRowsPerBlock * RPT, n_rows, inc, pos,
+      darcy_row_tile<DIM, NB, NP, NQ, kRowsPerBlock, R, GEO, RPT, RS_ONLY>(t * kRowsPerBlock * RPT, n_rows, inc, pos,
                                                                   rowptr, signs, cells, coords, tab, kinv, ks_e,
                                                                   ks_q, f, fs_e, fs_q, vals, rhs, st, sv, bc,
                                                                   first, geo);
@@ -846,6 +865,19 @@ __attribute__((amdgpu_waves_per_eu(batched_min_waves<KD>(), 8))) void k_darcy_ro
   }
 }
 
+// Blocks of a row kernel that the device holds at once (every GPU the library runs on is alike).
+static int resident_blocks(const void* kernel) {
+  int dev = 0, cus = 0, per_cu = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kRowsPerBlock, 0) != hipSuccess || cus < 1 ||
+      per_cu < 1) {
+    (void)hipGetLastError();
+    return 2048;
+  }
+  return cus * per_cu;
+}
+
 template <int DIM, int NB, int NP, int NQ, typename R>
 static int launch_darcy_rows(int n_rows, const int32_t* inc, const uint8_t* pos,
                              const int32_t* rowptr, const uint32_t* signs, const int32_t* cells,
@@ -858,23 +890,35 @@ static int launch_darcy_rows(int n_rows, const int32_t* inc, const uint8_t* pos,
                              const int32_t* tile_map = nullptr, int n_map = 0) {
   const DarcyRowBc<R> bc{n_bc, facet, combo, static_cast<const R*>(trace), static_cast<const R*>(fw),
                          static_cast<const R*>(pD), bc_rows};
-  // one slot per block for the lowest-order elements; a persistent grid (8 blocks per
-  // CU of 256, a multiple of the 8 XCDs) for the larger tables
+  // one slot per block for the lowest-order elements; a persistent grid for the larger tables
   const int n_slots = tile_map ? n_map : grid_for(n_rows, kRowsPerBlock * row_kernel_rpt<NB, R>());
-  const int grid = NB <= 4 ? n_slots : std::min(n_slots, 2048);
-  if (grid == 0) return NFX_OK;
+  if (n_slots == 0) return NFX_OK;
+  const auto launch = [&](auto kernel, int resident, const R* metric) {
+    hipLaunchKernelGGL(kernel, dim3(NB <= 4 ? n_slots : std::min(n_slots, resident)), dim3(kRowsPerBlock), 0, s,
+                       n_rows, inc, pos, rowptr, signs, cells, static_cast<const R*>(coords),
+                       static_cast<const R*>(tab), static_cast<const R*>(kinv), kse, ksq, static_cast<const R*>(f),
+                       fse, fsq, static_cast<R*>(vals), static_cast<R*>(rhs), bc, metric, tile_map, n_map);
+  };
+  const R* metric = static_cast<const R*>(geo);
+  if constexpr (NB > 4) {
+    // one coefficient per element: only the reference tensors in LDS (RT2: 25.6 KB a block instead of
+    // 32.3, and 116 registers instead of 166; 6 blocks a CU instead of 5: 42.5 us instead of 45.8), and as
+    // many blocks as are resident at once: on 41,154 tetrahedra, 4,227 tiles, 36.0 us with these 1,536
+    // blocks, 39.3 with 1,280, 41.3 with 2,048 (a third of them start when the others end), 37.4 with one
+    // tile a block. The sums over quadrature points are uneven from tile to tile: 105 us with 2,048
+    // blocks, 122 so.
+    if (geo && ksq == 0 && fsq == 0) {
+      constexpr auto kernel = k_darcy_rows<DIM, NB, NP, NQ, R, true, true>;
+      static const int resident = resident_blocks((const void*)kernel);
+      launch(kernel, resident, metric);
+      NFX_LAUNCH_CHECK();
+      return NFX_OK;
+    }
+  }
   if (geo)
-    hipLaunchKernelGGL((k_darcy_rows<DIM, NB, NP, NQ, R, true>), dim3(grid), dim3(kRowsPerBlock), 0, s, n_rows, inc,
-                       pos, rowptr, signs, cells, static_cast<const R*>(coords), static_cast<const R*>(tab),
-                       static_cast<const R*>(kinv), kse, ksq, static_cast<const R*>(f), fse, fsq,
-                       static_cast<R*>(vals), static_cast<R*>(rhs), bc, static_cast<const R*>(geo), tile_map,
-                       n_map);
+    launch(k_darcy_rows<DIM, NB, NP, NQ, R, true>, 2048, metric);
   else
-    hipLaunchKernelGGL((k_darcy_rows<DIM, NB, NP, NQ, R, false>), dim3(grid), dim3(kRowsPerBlock), 0, s, n_rows,
-                       inc, pos, rowptr, signs, cells, static_cast<const R*>(coords), static_cast<const R*>(tab),
-                       static_cast<const R*>(kinv), kse, ksq, static_cast<const R*>(f), fse, fsq,
-                       static_cast<R*>(vals), static_cast<R*>(rhs), bc, static_cast<const R*>(nullptr), tile_map,
-                       n_map);
+    launch(k_darcy_rows<DIM, NB, NP, NQ, R, false>, 2048, nullptr);
   NFX_LAUNCH_CHECK();
   return NFX_OK;
 }
