@@ -215,35 +215,6 @@ __global__ __launch_bounds__(256) void k_gnn_layer(int E, const int32_t* __restr
 
 // Heads: o_p = h_p.ud + cd, o_pj = a_pj ((h_p + h_q).ue + ce);
 // Wd = (omega0 + o_p) / S_pp, Wo_pj = o_pj / sqrt(S_pp S_qq).
-__global__ void k_gnn_heads(int E, const int32_t* __restrict__ nbr, const float* __restrict__ a,
-                            const uint16_t* __restrict__ th16, const float* __restrict__ th32,
-                            const uint16_t* __restrict__ h, const double* __restrict__ sdiag,
-                            float* __restrict__ Wd, float* __restrict__ Wo) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= E) return;
-  const uint16_t* hp = h + (int64_t)p * kW;
-  float od = 0.f;
-  for (int c = 0; c < kW; ++c) od += bf2f(hp[c]) * bf2f(th16[kOffUd + c]);
-  od += th32[kOffCd];
-  const double dp = sdiag[p];
-  Wd[p] = float((kOmega0 + od) / dp);
-  for (int j = 0; j < 4; ++j) {
-    const int q = nbr[4 * p + j];
-    if (q < 0) {
-      Wo[4 * p + j] = 0.f;
-      continue;
-    }
-    const uint16_t* hq = h + (int64_t)q * kW;
-    float s = 0.f;
-    for (int c = 0; c < kW; ++c) s += (bf2f(hp[c]) + bf2f(hq[c])) * bf2f(th16[kOffUe + c]);
-    const float oe = a[4 * p + j] * (s + th32[kOffCe]);
-    Wo[4 * p + j] = float(oe / sqrt(dp * sdiag[q]));
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Backward (FP32). Weight-gradient partials per block, summed in a fixed order.
-// ---------------------------------------------------------------------------
 // Rows of 64 channels are read 16 bytes a lane; the types carry the element's alignment
 // only (the hardware takes an unaligned global access), so any base pointer is allowed.
 typedef float f4u_t __attribute__((ext_vector_type(4), aligned(4)));
@@ -257,6 +228,54 @@ __device__ __forceinline__ void unpack8(const h8u_t& v, float (&o)[8]) {
   }
 }
 
+// Eight lanes a cell, eight channels each (one 16-byte load of the cell's row and of each neighbour's),
+// sums by a fixed butterfly. A thread per cell walked 5 x 64 channels in two-byte loads with one wave on
+// most CUs: 17.8 us at 24,576 cells, 4.2 here.
+__global__ __launch_bounds__(256) void k_gnn_heads(int E, const int32_t* __restrict__ nbr, const float* __restrict__ a,
+                                                   const uint16_t* __restrict__ th16, const float* __restrict__ th32,
+                                                   const uint16_t* __restrict__ h, const double* __restrict__ sdiag,
+                                                   float* __restrict__ Wd, float* __restrict__ Wo) {
+  static_assert(kW == 64, "eight lanes of eight channels");
+  const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  const int p = (int)(t >> 3), l = (int)(t & 7), c = 8 * l;
+  if (p >= E) return;  // whole groups of eight leave
+  float hp[8], hq[8], ud[8], ue[8], od = 0.f, s[4] = {0.f, 0.f, 0.f, 0.f};
+  int q[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) q[j] = nbr[4 * p + j];
+  h8u_t raw[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) raw[j] = *reinterpret_cast<const h8u_t*>(h + (int64_t)(q[j] >= 0 ? q[j] : p) * kW + c);
+  unpack8(*reinterpret_cast<const h8u_t*>(h + (int64_t)p * kW + c), hp);
+  unpack8(*reinterpret_cast<const h8u_t*>(th16 + kOffUd + c), ud);
+  unpack8(*reinterpret_cast<const h8u_t*>(th16 + kOffUe + c), ue);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) od += hp[i] * ud[i];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    unpack8(raw[j], hq);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) s[j] += (hp[i] + hq[i]) * ue[i];
+  }
+#pragma unroll
+  for (int off = 1; off < 8; off <<= 1) {
+    od += __shfl_xor(od, off, 8);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) s[j] += __shfl_xor(s[j], off, 8);
+  }
+  const double dp = sdiag[p];
+  if (l == 4) Wd[p] = float((kOmega0 + (od + th32[kOffCd])) / dp);
+  if (l < 4) {
+    const int ql = l == 0 ? q[0] : l == 1 ? q[1] : l == 2 ? q[2] : q[3];
+    const float sl = l == 0 ? s[0] : l == 1 ? s[1] : l == 2 ? s[2] : s[3];
+    const float oe = a[4 * p + l] * (sl + th32[kOffCe]);
+    Wo[4 * p + l] = ql < 0 ? 0.f : float(oe / sqrt(dp * sdiag[ql]));
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Backward (FP32). Weight-gradient partials per block, summed in a fixed order.
+// ---------------------------------------------------------------------------
 __device__ __forceinline__ float4_t mfma_f32_4(float a, float b, float4_t c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
@@ -629,38 +648,56 @@ __global__ void k_ell_spmm(int E, int ns, const int32_t* __restrict__ nbr, const
 }
 
 // gamma_d[p] = sum_s w_s Su_p Se_p; gamma_o[p][j] = sum_s w_s (Su_p Se_q + Su_q Se_p)
-__global__ void k_smoother_grad(int E, int ns, const int32_t* __restrict__ nbr,
-                                const float* __restrict__ Su, const float* __restrict__ Se,
-                                const float* __restrict__ w, float* __restrict__ gd,
-                                float* __restrict__ go) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= E) return;
+// Four lanes a cell share the samples (sums by a fixed butterfly): a thread per cell over all of them took
+// 19.0 us at 24,576 cells and 12 samples, 5.5 here.
+__global__ __launch_bounds__(256) void k_smoother_grad(int E, int ns, const int32_t* __restrict__ nbr,
+                                                       const float* __restrict__ Su, const float* __restrict__ Se,
+                                                       const float* __restrict__ w, float* __restrict__ gd,
+                                                       float* __restrict__ go) {
+  const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  const int p = (int)(t >> 2), l = (int)(t & 3);
+  if (p >= E) return;  // whole groups of four leave
   float d = 0.f, o[4] = {0.f, 0.f, 0.f, 0.f};
   int q[4];
+#pragma unroll
   for (int j = 0; j < 4; ++j) q[j] = nbr[4 * p + j];
-  for (int s = 0; s < ns; ++s) {
+#pragma unroll 4
+  for (int s = l; s < ns; s += 4) {
     const float* su = Su + (int64_t)s * E;
     const float* se = Se + (int64_t)s * E;
-    const float ws = w[s], sup = su[p] * ws, sep = se[p] * ws;
-    d += sup * se[p];
-    for (int j = 0; j < 4; ++j)
-      if (q[j] >= 0) o[j] += sup * se[q[j]] + sep * su[q[j]];
+    const float ws = w[s], sup = su[p] * ws, e = se[p], sep = e * ws;
+    d += sup * e;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int n = q[j] >= 0 ? q[j] : p;
+      const float c = sup * se[n] + sep * su[n];
+      o[j] += q[j] >= 0 ? c : 0.f;
+    }
   }
-  gd[p] = d;
-  for (int j = 0; j < 4; ++j) go[4 * p + j] = o[j];
+#pragma unroll
+  for (int off = 1; off < 4; off <<= 1) {
+    d += __shfl_xor(d, off, 4);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) o[j] += __shfl_xor(o[j], off, 4);
+  }
+  if (l == 0) gd[p] = d;
+  go[4 * p + l] = l == 0 ? o[0] : l == 1 ? o[1] : l == 2 ? o[2] : o[3];
 }
 
-// C[s][a] = sum over members p of aggregate a (member order) of X[s][p]
-__global__ void k_agg_sum(int n_agg, int ns, int E, const int32_t* __restrict__ agg_ptr,
-                          const int32_t* __restrict__ agg_mem, const float* __restrict__ X,
-                          float* __restrict__ C) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+// C[s][a] = sum over members p of aggregate a of X[s][p]: a wave per (s, a), a fixed butterfly (a thread
+// walked the ~48 members in 15.4 us for 512 aggregates and 12 samples, 3.5 here)
+__global__ __launch_bounds__(256) void k_agg_sum(int n_agg, int ns, int E, const int32_t* __restrict__ agg_ptr,
+                                                 const int32_t* __restrict__ agg_mem, const float* __restrict__ X,
+                                                 float* __restrict__ C) {
+  const int64_t i = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 6;
   if (i >= (int64_t)n_agg * ns) return;
   const int64_t s = i / n_agg;
-  const int ag = int(i % n_agg);
+  const int ag = int(i % n_agg), lane = threadIdx.x & 63;
   float acc = 0.f;
-  for (int k = agg_ptr[ag]; k < agg_ptr[ag + 1]; ++k) acc += X[s * E + agg_mem[k]];
-  C[i] = acc;
+  for (int k = agg_ptr[ag] + lane; k < agg_ptr[ag + 1]; k += 64) acc += X[s * E + agg_mem[k]];
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
+  if (lane == 0) C[i] = acc;
 }
 
 // Dense coarse operator row a: Ac[a][agg(q)] += S_pq for members p of a (FP64, one wave per
@@ -1251,7 +1288,7 @@ int nfx_gnn_forward(int E, const int32_t* nbr, const float* a, const float* x, c
                        h + l * EW, m + l * EW, z + (l + 1) * EW, h + (l + 1) * EW);
     NFX_LAUNCH_CHECK();
   }
-  hipLaunchKernelGGL(k_gnn_heads, dim3(grid_for(E, 256)), dim3(256), 0, st, E, nbr, a, theta16, theta32,
+  hipLaunchKernelGGL(k_gnn_heads, dim3(grid_for(8 * (int64_t)E, 256)), dim3(256), 0, st, E, nbr, a, theta16, theta32,
                      h + kLayers * EW, sdiag, Wd, Wo);
   NFX_LAUNCH_CHECK();
   return NFX_OK;
@@ -1315,7 +1352,7 @@ int nfx_smoother_grad(int E, int ns, const int32_t* nbr, const float* Su, const 
   NFX_REQUIRE(E >= 0 && ns >= 0, "nfx_smoother_grad: negative size");
   if (E == 0) return NFX_OK;
   NFX_REQUIRE(nbr && Su && Se && w && gamma_d && gamma_o, "nfx_smoother_grad: null pointer");
-  hipLaunchKernelGGL(k_smoother_grad, dim3(grid_for(E, 256)), dim3(256), 0, (hipStream_t)stream, E, ns, nbr,
+  hipLaunchKernelGGL(k_smoother_grad, dim3(grid_for(4 * (int64_t)E, 256)), dim3(256), 0, (hipStream_t)stream, E, ns, nbr,
                      Su, Se, w, gamma_d, gamma_o);
   NFX_LAUNCH_CHECK();
   return NFX_OK;
@@ -1326,7 +1363,7 @@ int nfx_agg_sum(int n_agg, int ns, int E, const int32_t* agg_ptr, const int32_t*
   NFX_REQUIRE(n_agg >= 0 && ns >= 0 && E >= 0, "nfx_agg_sum: negative size");
   if ((int64_t)n_agg * ns == 0) return NFX_OK;
   NFX_REQUIRE(agg_ptr && agg_mem && X && C, "nfx_agg_sum: null pointer");
-  hipLaunchKernelGGL(k_agg_sum, dim3(grid_for((int64_t)n_agg * ns, 256)), dim3(256), 0, (hipStream_t)stream,
+  hipLaunchKernelGGL(k_agg_sum, dim3(grid_for((int64_t)n_agg * ns * 64, 256)), dim3(256), 0, (hipStream_t)stream,
                      n_agg, ns, E, agg_ptr, agg_mem, X, C);
   NFX_LAUNCH_CHECK();
   return NFX_OK;
