@@ -14,7 +14,7 @@ struct BmGridBlock {
 };
 
 // Launch plan and work space of a batch. An instance's block count follows from its own size, so its
-// sums, and its result, are the same whatever else is in the batch.
+// sums, and its result, are the same in every batch that is resident.
 struct BmGrid {
   char *dev = nullptr, *host = nullptr;  // one allocation each
   std::vector<int> wave_of;    // launch of each instance, -1: not resident
@@ -28,7 +28,8 @@ struct BmGrid {
   double* h_tol = nullptr;
 };
 
-constexpr int kBmRanges = 12;  // per preconditioner group: first, end and run count of cells and of flux blocks
+// per preconditioner group: first, end and run count of cells and of flux blocks; then the aggregates
+constexpr int kBmRanges = 13;
 
 // Plans the launches and allocates (nothing resident when the device or the sizes do not allow it).
 int bm_grid_create(BmGrid* g, int n_inst, const nfx_minres_batch_item* items, const nfx_minres_batch_item* d_items,

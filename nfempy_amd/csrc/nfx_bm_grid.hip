@@ -54,8 +54,10 @@ __global__ __launch_bounds__(256) void k_bm_grid_zero(int n, int32_t* p) {
 }
 
 // runs of equal instance in a group's cells (what 0) or flux blocks (1): first, end, number of runs
+// (and, of cells, the instance's aggregates)
 __global__ __launch_bounds__(256) void k_bm_ranges(int n, const int32_t* __restrict__ inst, int n_inst, int group,
-                                                   int what, int32_t* __restrict__ ranges) {
+                                                   int what, const int32_t* __restrict__ agg_of,
+                                                   const int32_t* __restrict__ alen, int32_t* __restrict__ ranges) {
   const int c = blockIdx.x * 256 + threadIdx.x;
   if (c >= n) return;
   const int i = inst[c];
@@ -64,6 +66,7 @@ __global__ __launch_bounds__(256) void k_bm_ranges(int n, const int32_t* __restr
   if (c == 0 || inst[c - 1] != i) {
     r[0] = c;
     atomicAdd(r + 2, 1);
+    if (what == 0) atomicMax(ranges + (int64_t)i * kBmRanges + 12, alen[agg_of[c]]);
   }
   if (c == n - 1 || inst[c + 1] != i) r[1] = c + 1;
 }
@@ -637,9 +640,14 @@ int bm_grid_solve(BmGrid* g, int n_inst, int64_t n_total, const nfx_minres_batch
   const int waves = (int)g->wave_at.size() - 1;
   std::vector<char> runs(std::max(waves, 1), 0);
   bool any = false;
+  // all or none: beside instances that have to iterate stepwise the others cost little there and a launch
+  // each here (32 instances up to 16 x 16 x 16 cubes: 79.5 ms stepwise, 94.5 ms split)
   for (int i = 0; i < n_inst; ++i)
-    if (h_mode[i] == 0 && g->wave_of[i] >= 0) any = runs[g->wave_of[i]] = 1;
-  if (!any || n_total > INT32_MAX) return NFX_OK;
+    if (h_mode[i] == 0) {
+      if (g->wave_of[i] < 0) return NFX_OK;
+      any = runs[g->wave_of[i]] = 1;
+    }
+  if (!any || n_total > INT32_MAX || grid_refused()) return NFX_OK;
 
   for (int i = 0; i < n_inst; ++i) g->h_tol[i] = tol[i];
   NFX_CHECK_HIP(hipMemcpyAsync(g->tol, g->h_tol, sizeof(double) * n_inst, hipMemcpyHostToDevice, st));
@@ -663,13 +671,22 @@ int bm_grid_solve(BmGrid* g, int n_inst, int64_t n_total, const nfx_minres_batch
   for (int q = 0; q < a.n_groups; ++q) {
     a.pc[q] = pc[q];
     hipLaunchKernelGGL(k_bm_ranges, dim3(grid_for(pc[q].n_cells, 256)), dim3(256), 0, st, pc[q].n_cells,
-                       pc[q].cell_inst, n_inst, q, 0, g->ranges);
+                       pc[q].cell_inst, n_inst, q, 0, pc[q].agg_of, pc[q].alen, g->ranges);
     if (pc[q].n_fb > 0)
       hipLaunchKernelGGL(k_bm_ranges, dim3(grid_for(pc[q].n_fb, 256)), dim3(256), 0, st, pc[q].n_fb, pc[q].fb_inst,
-                         n_inst, q, 1, g->ranges);
+                         n_inst, q, 1, nullptr, nullptr, g->ranges);
   }
   NFX_LAUNCH_CHECK();
+  if (a.n_groups) {
+    // an instance with too many aggregates for the cycle here: the batch stays together
+    std::vector<int32_t> r((size_t)n_inst * kBmRanges);
+    NFX_CHECK_HIP(hipMemcpyAsync(r.data(), g->ranges, sizeof(int32_t) * r.size(), hipMemcpyDeviceToHost, st));
+    NFX_CHECK_HIP(hipStreamSynchronize(st));
+    for (int i = 0; i < n_inst; ++i)
+      if (h_mode[i] == 0 && r[(size_t)i * kBmRanges + 12] > kBmGridAgg) return NFX_OK;
+  }
   bool first = true;
+  int runs_until = waves;
   for (int w = 0; w < waves; ++w) {
     if (!runs[w]) continue;
     const int nblk = g->wave_at[w + 1] - g->wave_at[w];
@@ -680,12 +697,18 @@ int bm_grid_solve(BmGrid* g, int n_inst, int64_t n_total, const nfx_minres_batch
     first = false;
     a.blocks = g->blocks + g->wave_at[w];
     void* args[] = {&a};
-    NFX_CHECK_HIP(hipLaunchCooperativeKernel((const void*)k_bm_grid, dim3(nblk), dim3(kT), args, kGridLdsBytes, st));
+    if (hipLaunchCooperativeKernel((const void*)k_bm_grid, dim3(nblk), dim3(kT), args, kGridLdsBytes, st) !=
+        hipSuccess) {
+      (void)hipGetLastError();  // refused (nothing ran): the stepwise kernels take this and the later launches
+      grid_note_refusal();
+      runs_until = w;
+      break;
+    }
   }
   NFX_CHECK_HIP(hipMemcpyAsync(g->h_res, g->res, sizeof(GridResult) * n_inst, hipMemcpyDeviceToHost, st));
   NFX_CHECK_HIP(hipStreamSynchronize(st));
   for (int i = 0; i < n_inst; ++i)
-    if (h_mode[i] == 0 && g->wave_of[i] >= 0 && g->h_res[i].status == 0) {
+    if (h_mode[i] == 0 && g->wave_of[i] >= 0 && g->wave_of[i] < runs_until && g->h_res[i].status == 0) {
       (*done)[i] = 1;
       iters[i] = g->h_res[i].iters;
     }

@@ -462,11 +462,18 @@ int el_grid_blocks(int max_blocks, const nfx_elasticity_tg* pc, int n_blocks) {
 int el_grid_solve(const MinresGrid* g, int nblk, int n, int n_blocks, const int32_t* brp, const int32_t* bci,
                   const float* bva, const nfx_elasticity_tg* pc, const float* rhs, float* x, float* vec, double tol,
                   int maxit, int* iters, int* status, hipStream_t st) {
+  *status = 1;
+  if (grid_refused()) return NFX_OK;
   hipLaunchKernelGGL(k_el_grid_clear, dim3(grid_for(kGridSlotWords, 256)), dim3(256), 0, st, g->slots, g->res);
   NFX_LAUNCH_CHECK();
   ElGridArgs a{n, n_blocks, nblk, maxit, kGridLdsBytes, brp, bci, bva, *pc, rhs, x, vec, tol, g->slots, g->res};
   void* args[] = {&a};
-  NFX_CHECK_HIP(hipLaunchCooperativeKernel((const void*)k_el_grid, dim3(nblk), dim3(kT), args, kGridLdsBytes, st));
+  if (hipLaunchCooperativeKernel((const void*)k_el_grid, dim3(nblk), dim3(kT), args, kGridLdsBytes, st) != hipSuccess) {
+    (void)hipGetLastError();  // refused (nothing ran): the stepwise kernels take it
+    grid_note_refusal();
+    *status = 1;
+    return NFX_OK;
+  }
   NFX_CHECK_HIP(hipMemcpyAsync(g->h_res, g->res, sizeof(GridResult), hipMemcpyDeviceToHost, st));
   NFX_CHECK_HIP(hipStreamSynchronize(st));
   *iters = g->h_res->iters;

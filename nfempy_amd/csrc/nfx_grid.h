@@ -23,6 +23,13 @@ namespace nfx {
 // 1,024 against 512 threads, us an iteration of MINRES: 4.5 / 4.5 at 5,184 rows (30 k entries), 7.7 / 9.9 at
 // 41,088 rows (1.06 M entries) and 8.7 / 11.3 at 252,288 rows (1.9 M): more rows in flight beside the waits
 constexpr int kGridThreads = 1024;
+
+// A device gives the resources of cooperative launches to one process at a time; a launch in another is
+// refused, after ~35 ms. The callers then take the stepwise kernels, and for kGridRetrySeconds they do not
+// ask again (nfx_minres_grid.hip).
+constexpr int kGridRetrySeconds = 10;
+bool grid_refused();
+void grid_note_refusal();
 constexpr int kGridMaxBlocks = 256;
 constexpr int kGridCopies = 8;
 constexpr int kGridBlockWords = 2 * kGridCopies * 2;  // 64-bit words of slots per block

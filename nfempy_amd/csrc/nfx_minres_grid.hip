@@ -9,6 +9,8 @@
 // An iteration took 10.1 us as two launches and 4.5 us here at 5,184 rows (triangles, degree 1), 14.0
 // and 7.7 at 41,088 rows (tetrahedra, degree 2), 18.7 and 8.7 at 252,288 rows (tetrahedra, degree 1).
 #include <algorithm>
+#include <atomic>
+#include <chrono>
 #include <cstdint>
 
 #include "nfx_minres_grid.h"
@@ -206,6 +208,19 @@ __global__ __launch_bounds__(kGridThreads) void k_minres_grid(MinresGridArgs a) 
   if (blockIdx.x == 0 && t == 0) a.res->iters = k > 1 ? k - 1 : 1;
 }
 
+namespace {
+std::atomic<int64_t> g_retry_at{0};  // steady clock, ns; any device of the process
+int64_t grid_clock() {
+  return std::chrono::duration_cast<std::chrono::nanoseconds>(std::chrono::steady_clock::now().time_since_epoch())
+      .count();
+}
+}  // namespace
+
+bool grid_refused() { return g_retry_at.load(std::memory_order_relaxed) > grid_clock(); }
+void grid_note_refusal() {
+  g_retry_at.store(grid_clock() + (int64_t)kGridRetrySeconds * 1000000000, std::memory_order_relaxed);
+}
+
 // Resident blocks that the device allows (0: no cooperative launch, or too little LDS).
 int minres_grid_capacity() {
   int dev = 0, coop = 0, cus = 0, per_cu = 0;
@@ -249,6 +264,8 @@ int minres_grid_solve(MinresGrid* g, int nblk, int lanes, int n, const int32_t* 
                       const float* sign, const int32_t* prp, const int32_t* pci, const float* pva, const float* rhs,
                       float* x, float* z, double tol, int maxit, int* iters, int* status, hipStream_t st) {
   NFX_REQUIRE(nblk > 0 && nblk <= g->max_blocks, "minres_grid_solve: blocks");
+  *status = 1;
+  if (grid_refused()) return NFX_OK;
   hipLaunchKernelGGL(k_grid_clear, dim3(grid_for(kGridSlotWords, 256)), dim3(256), 0, st, g->slots, g->res);
   NFX_LAUNCH_CHECK();
   MinresGridArgs a{n, nblk, maxit, kGridLdsBytes, rp, ci, va, sign, prp, pci, pva, rhs, x, z, tol, g->slots, g->res};
@@ -256,7 +273,12 @@ int minres_grid_solve(MinresGrid* g, int nblk, int lanes, int n, const int32_t* 
   const void* f = lanes == 16  ? (const void*)k_minres_grid<16>
                   : lanes == 8 ? (const void*)k_minres_grid<8>
                                : (const void*)k_minres_grid<4>;
-  NFX_CHECK_HIP(hipLaunchCooperativeKernel(f, dim3(nblk), dim3(kGridThreads), args, kGridLdsBytes, st));
+  if (hipLaunchCooperativeKernel(f, dim3(nblk), dim3(kGridThreads), args, kGridLdsBytes, st) != hipSuccess) {
+    (void)hipGetLastError();  // refused (nothing ran): the stepwise kernels take it
+    grid_note_refusal();
+    *status = 1;
+    return NFX_OK;
+  }
   NFX_CHECK_HIP(hipMemcpyAsync(g->h_res, g->res, sizeof(GridResult), hipMemcpyDeviceToHost, st));
   NFX_CHECK_HIP(hipStreamSynchronize(st));
   *iters = g->h_res->iters;

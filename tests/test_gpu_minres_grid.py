@@ -114,18 +114,24 @@ def test_exact_breakdown_is_finite():
 
 @pytest.mark.parametrize("pc", ["diag", "twogrid", "learned"])
 def test_batch_over_resident_sizes(pc):
-    """Instances of one block, of many, more blocks than fit one launch, and (11 cubed: 216 aggregates)
-    one that the two-grid cycle leaves to the stepwise kernels: FP64 residuals, and each instance bitwise
-    what it is alone (its block count follows from its own size)."""
+    """Instances of one block, of many, more blocks than fit one launch: FP64 residuals, and each instance
+    bitwise what it is alone (its block count follows from its own size); then, with an instance that the
+    two-grid cycle leaves to the stepwise kernels (11 cubed: 216 aggregates), the whole batch there."""
     import torch
 
     from nfempy_amd.batch import DarcyBatch
 
-    specs = [(2, 1), (9, 2), (11, 1), (5, 2), (9, 2), (7, 1), (1, 2), (9, 2)]
+    specs = [(2, 1), (9, 2), (5, 2), (9, 2), (7, 1), (1, 2), (9, 2), (11, 1)]
     b = DarcyBatch(specs, seed=4, workers=1)
     b.assemble()
     print(f"[minres grid] batch {pc}", flush=True)
-    xs, infos, _ = b.solve_batched(rtol=1e-8, pc=pc)
+    mixed, mixed_infos, _ = b.solve_batched(rtol=1e-8, pc=pc)
+    xs, infos, _ = b.solve_batched(list(range(7)), rtol=1e-8, pc=pc)
+    xs.append(mixed[7])
+    infos.append(mixed_infos[7])
+    for i in range(7):  # both within rtol of the solution, times the conditioning
+        assert mixed_infos[i]["converged"]
+        assert float((mixed[i] - xs[i]).norm() / xs[i].norm()) <= 1e-6
     for i in range(len(specs)):
         assert infos[i]["converged"], (i, infos[i])
         y = b.fp64_system(i)
