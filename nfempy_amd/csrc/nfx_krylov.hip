@@ -7,6 +7,8 @@
 // iterations, so an iteration is two kernel launches:
 //   A(k): x/w update of iteration k-1, y = D A z / beta - (beta/oldb) r1, alpha = v.y
 //   B(k): y -= (alpha/beta) r2, z = P^-1 y, beta' = sqrt(y.z), Givens update
+// Systems that fit the CUs' LDS run whole inner solves as one launch instead (nfx_minres_grid.hip,
+// nfx_bm_grid.hip, nfx_el_grid.hip); what follows serves the others and is where those fall back to.
 #include <algorithm>
 #include <cmath>
 #include <vector>
