@@ -532,7 +532,8 @@ int nfx_batch_tg_apply(int n_groups, const nfx_batch_tg* pc, const int32_t* d_mo
                        void* stream);
 /* Attach (n_groups 1 or 2, of different nb) or detach (0) two-grid groups to a batched MINRES: each application
  * of its preconditioner then runs the diagonal one and, on the groups' rows, the cycle. The
- * descriptors are copied; the arrays they point to must outlive the solves. */
+ * descriptors are copied; the arrays they point to must outlive the solves. NFX_E_INVALID for a group with a
+ * missing array, or with smoother couplings and nb = 4. */
 int nfx_minres_batch_set_pc(nfx_minres_batch* s, int n_groups, const nfx_batch_tg* h_groups);
 
 /* ---- sort-based numbering (cold path) ---------------------------------------

@@ -566,13 +566,19 @@ int check_desc(const nfx_batch_tg* pc) {
 
 }  // namespace
 
-int batch_tg_apply(const nfx_batch_tg* pc, int n_groups, const int32_t* mode, const float* r, float* z,
-                   hipStream_t st) {
-  NFX_REQUIRE(pc && (n_groups == 1 || n_groups == 2), "nfx_batch_tg_apply: one or two groups");
+int batch_tg_check(const nfx_batch_tg* pc, int n_groups) {
   for (int g = 0; g < n_groups; ++g) {
     const int rc = check_desc(pc + g);
     if (rc) return rc;
   }
+  return NFX_OK;
+}
+
+int batch_tg_apply(const nfx_batch_tg* pc, int n_groups, const int32_t* mode, const float* r, float* z,
+                   hipStream_t st) {
+  NFX_REQUIRE(pc && (n_groups == 1 || n_groups == 2), "nfx_batch_tg_apply: one or two groups");
+  const int rc = batch_tg_check(pc, n_groups);
+  if (rc) return rc;
   if (n_groups == 1)
     return pc->nb == 1 ? apply_pair<1, 1>(pc[0], nullptr, mode, r, z, st) : apply_pair<4, 4>(pc[0], nullptr, mode, r, z, st);
   NFX_REQUIRE(pc[0].nb != pc[1].nb, "nfx_batch_tg_apply: two groups need different nb");

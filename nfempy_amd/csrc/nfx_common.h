@@ -89,5 +89,7 @@ int el_twogrid_apply_scaled(const nfx_elasticity_tg* pc, const float* r, float* 
 // in shared launches (nfx_batch_tg_apply); mode as there.
 int batch_tg_apply(const nfx_batch_tg* pc, int n_groups, const int32_t* mode, const float* r, float* z,
                    hipStream_t stream);
+// NFX_E_INVALID for a group that no kernel may read: set_pc and every route of a solve ask first.
+int batch_tg_check(const nfx_batch_tg* pc, int n_groups);
 
 }  // namespace nfx

@@ -105,6 +105,9 @@ __device__ __forceinline__ void el_post(int m, int n_cells, const int32_t* __res
   }
 }
 
+// NFX_E_INVALID for a descriptor that no kernel may read: every route of a solve asks first.
+int el_tg_check(const nfx_elasticity_tg* pc);
+
 // The middle of the cycle on the device work buffers: rc = P^T (r - S x1) and y = Ainv rc
 // (x1 must be in the work buffer already).
 int el_tg_launch_mid(const nfx_elasticity_tg* pc, const float* r, hipStream_t st);

@@ -236,7 +236,7 @@ __global__ __launch_bounds__(kTgBlock) void k_el_tg_post(int n_cells, int ns, in
 
 using namespace nfx;
 
-static int el_tg_check(const nfx_elasticity_tg* pc) {
+int nfx::el_tg_check(const nfx_elasticity_tg* pc) {
   NFX_REQUIRE(pc, "nfx_elasticity_tg: null descriptor");
   const int ns = pc->n_s, nu = pc->n_u, E = pc->n_cells, n_agg = pc->n_agg;
   NFX_REQUIRE(ns >= 0 && ns % 9 == 0 && nu == 3 * E && E > 0 && n_agg > 0, "nfx_elasticity_tg: sizes");

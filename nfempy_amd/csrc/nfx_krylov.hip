@@ -876,6 +876,8 @@ extern "C" int nfx_solve_minres_ir_tg(nfx_solver* s, const int32_t* d_rowptr, co
     hipLaunchKernelGGL(k_to_f32, dim3(g), dim3(kBlock), 0, s->stream, n, s->r64, nullptr, rn, rf);
     NFX_LAUNCH_CHECK();
     int it = 0;
+    rc = el_tg_check(pc);
+    if (rc) return rc;
     if (grid_blocks) {
       int status = 0;
       rc = el_grid_solve(&s->grid, grid_blocks, n, s->b3_nblk, s->b3_rp, s->b3_ci, s->b3_va, pc, rf, dx, s->buf,
@@ -1345,11 +1347,8 @@ extern "C" int nfx_minres_batch_set_pc(nfx_minres_batch* s, int n_groups, const 
   NFX_REQUIRE(n_groups <= 2 && (n_groups < 2 || h_groups[0].nb != h_groups[1].nb),
               "nfx_minres_batch_set_pc: at most two groups, of different nb");
   std::vector<nfx_batch_tg> g(h_groups, h_groups + n_groups);
-  for (const nfx_batch_tg& d : g) {
-    NFX_REQUIRE(d.nb == 1 || d.nb == 4, "nfx_minres_batch_set_pc: nb must be 1 or 4");
-    NFX_REQUIRE(d.n_cells > 0 && d.n_agg > 0 && d.cell_inst && d.prow && d.work,
-                "nfx_minres_batch_set_pc: incomplete group");
-  }
+  const int rc = nfx::batch_tg_check(g.data(), n_groups);
+  if (rc) return rc;
   s->pc.swap(g);
   return NFX_OK;
 }
@@ -1522,6 +1521,8 @@ extern "C" int nfx_solve_minres_batch_ir(nfx_minres_batch* s, const double* d_b,
     // instances that fit a few CUs as resident launches, the rest stepwise together
     std::vector<char> done;
     std::vector<int> resident(m, 0);
+    rc = nfx::batch_tg_check(s->pc.data(), (int)s->pc.size());
+    if (rc) return rc;
     rc = nfx::bm_grid_solve(&s->grid, m, N, s->items, s->mode, s->h_mode, s->pc, rf, dx, s->buf, s->buf + N * 10, tol.data(),
                             max_inner, resident.data(), &done, st);
     if (rc) return rc;
