@@ -52,7 +52,8 @@ extern "C" {
  * row assembly, packed positions and entry signs of the lowest-order rows; 0.4.0: in-tile
  * row offsets in the lowest-order position words, compact RT2 batched launch, degree 3;
  * 0.5.0: flux-row operator fields of nfx_twogrid_pc (flux_width, flux_col, flux_coef, appended
- * after tail_coef) and nfx_flux_sweep_coef). */
+ * after tail_coef) and nfx_flux_sweep_coef).
+ * 0.5.1: nfx_*_set_resident, nfx_*_resident_counts. */
 int nfx_version(void);
 /* Thread-local description of the last error on this thread. */
 const char* nfx_last_error(void);
@@ -350,6 +351,15 @@ int nfx_schur_diag64(int n_rows, int n_u, const int32_t* d_rowptr,
 typedef struct nfx_solver nfx_solver;
 int nfx_solver_create(nfx_solver** out, int n_rows, int nnz, void* stream);
 int nfx_solver_destroy(nfx_solver* s);
+/* Resident solves. An inner solve of a system that fits the compute units' local memory runs as one
+ * cooperative launch where the device gives one, stepwise (a few launches an iteration) otherwise; the two
+ * differ by roundings. launches: how many resident launches the object may still make (-1: any number, the
+ * default; 0: stepwise only). absent != 0 (for tests of what follows): launches leave out their last block,
+ * so that the others of its system give up waiting for it after half a second, as they do where the device
+ * does not run them all, and the solve goes on stepwise. h_counts (2 values), since creation: inner solves
+ * that ran resident, and those that were tried so and ran stepwise. */
+int nfx_solver_set_resident(nfx_solver* s, int64_t launches, int absent);
+int nfx_solver_resident_counts(const nfx_solver* s, int64_t* h_counts);
 /* Give the solver a 3 x 3 block CSR copy of the FP32 operator it is then called with
  * (n_rows a multiple of 3; block row R holds rows 3R .. 3R+2, d_browptr (n_rows/3 + 1),
  * d_bcol (n_blocks) block columns, d_bval 9 n_blocks values with entry (a, b) of block j
@@ -444,6 +454,9 @@ typedef struct nfx_minres_batch nfx_minres_batch;
 int nfx_minres_batch_create(nfx_minres_batch** out, int n_inst, const nfx_minres_batch_item* h_items,
                             void* stream);
 int nfx_minres_batch_destroy(nfx_minres_batch* s);
+/* As nfx_solver_set_resident and nfx_solver_resident_counts; the counts are of instances. */
+int nfx_minres_batch_set_resident(nfx_minres_batch* s, int64_t launches, int absent);
+int nfx_minres_batch_resident_counts(const nfx_minres_batch* s, int64_t* h_counts);
 /* Total rows of the batch (the length of d_b and d_x); a count, not a status. */
 int64_t nfx_minres_batch_rows(const nfx_minres_batch* s);
 /* Synchronous. Each refinement step of an instance stops its inner MINRES at the relative

@@ -86,6 +86,8 @@ SIGNATURES = {
     "nfx_schur_diag64": (c_int, [c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
     "nfx_solver_create": (c_int, [c_void_p, c_int, c_int, c_void_p]),
     "nfx_solver_destroy": (c_int, [c_void_p]),
+    "nfx_solver_set_resident": (c_int, [c_void_p, c_i64, c_int]),
+    "nfx_solver_resident_counts": (c_int, [c_void_p, c_void_p]),
     "nfx_solve_minres_ir": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                     c_void_p, c_void_p, c_void_p, c_void_p, c_double, c_double, c_int, c_int,
                                     c_void_p, c_void_p, c_void_p, c_int]),
@@ -117,6 +119,8 @@ SIGNATURES = {
     "nfx_minres_batch_create": (c_int, [c_void_p, c_int, c_void_p, c_void_p]),
     "nfx_minres_batch_destroy": (c_int, [c_void_p]),
     "nfx_minres_batch_rows": (c_i64, [c_void_p]),
+    "nfx_minres_batch_set_resident": (c_int, [c_void_p, c_i64, c_int]),
+    "nfx_minres_batch_resident_counts": (c_int, [c_void_p, c_void_p]),
     "nfx_minres_batch_set_pc": (c_int, [c_void_p, c_int, c_void_p]),
     "nfx_batch_tg_schur": (c_int, [c_int, c_int, c_int, c_int] + [c_void_p] * 11 + [c_void_p]),
     "nfx_batch_tg_schur_blk": (c_int, [c_int] + [c_void_p] * 13 + [c_void_p]),

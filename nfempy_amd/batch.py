@@ -336,6 +336,7 @@ class DarcyBatch:
         x, infos = mb.solve(b, rtol=rtol, inner_rtol=inner_rtol, max_inner=max_inner, max_outer=max_outer)
         t.cuda.synchronize()
         dt = time.perf_counter() - t0
+        self.last_resident = mb.resident_counts()
         mb.close()
         if tg is not None:
             for info in infos:

@@ -19,6 +19,7 @@ struct BmGrid {
   char *dev = nullptr, *host = nullptr;  // one allocation each
   std::vector<int> wave_of;    // launch of each instance, -1: not resident
   std::vector<int> wave_at;    // first block of each launch in blocks[], and the end
+  std::vector<char> tail;      // per launch: its last block is one of several of an instance
   BmGridBlock* blocks = nullptr;
   int32_t* ranges = nullptr;   // kBmRanges per instance
   grid_word* slots = nullptr;
@@ -26,6 +27,7 @@ struct BmGrid {
   double* tol = nullptr;       // per instance
   GridResult* h_res = nullptr; // pinned, per instance
   double* h_tol = nullptr;
+  GridControl control;
 };
 
 // per preconditioner group: first, end and run count of cells and of flux blocks; then the aggregates

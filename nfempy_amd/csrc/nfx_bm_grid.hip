@@ -42,12 +42,6 @@ struct BmGridArgs {
   GridResult* res;
 };
 
-__global__ __launch_bounds__(256) void k_bm_grid_clear(int64_t words, grid_word* slots, int n_inst, GridResult* res) {
-  const int64_t i = blockIdx.x * 256 + threadIdx.x;
-  if (i < words) slots[i] = 0;
-  if (i < n_inst && res) res[i] = GridResult{0, 0};
-}
-
 __global__ __launch_bounds__(256) void k_bm_grid_zero(int n, int32_t* p) {
   const int i = blockIdx.x * 256 + threadIdx.x;
   if (i < n) p[i] = 0;
@@ -622,6 +616,7 @@ int bm_grid_create(BmGrid* g, int n_inst, const nfx_minres_batch_item* items, co
   for (const auto& w : waves) {
     all.insert(all.end(), w.begin(), w.end());
     g->wave_at.push_back((int)all.size());
+    g->tail.push_back(w.back().nblk > 1);
   }
   if (!all.empty()) NFX_CHECK_HIP(hipMemcpy(g->blocks, all.data(), sizeof(BmGridBlock) * all.size(), hipMemcpyHostToDevice));
   return NFX_OK;
@@ -647,7 +642,7 @@ int bm_grid_solve(BmGrid* g, int n_inst, int64_t n_total, const nfx_minres_batch
       if (g->wave_of[i] < 0) return NFX_OK;
       any = runs[g->wave_of[i]] = 1;
     }
-  if (!any || n_total > INT32_MAX || grid_refused()) return NFX_OK;
+  if (!any || n_total > INT32_MAX || !g->control.launches || grid_refused()) return NFX_OK;
 
   for (int i = 0; i < n_inst; ++i) g->h_tol[i] = tol[i];
   NFX_CHECK_HIP(hipMemcpyAsync(g->tol, g->h_tol, sizeof(double) * n_inst, hipMemcpyHostToDevice, st));
@@ -690,28 +685,27 @@ int bm_grid_solve(BmGrid* g, int n_inst, int64_t n_total, const nfx_minres_batch
   for (int w = 0; w < waves; ++w) {
     if (!runs[w]) continue;
     const int nblk = g->wave_at[w + 1] - g->wave_at[w];
-    const int64_t words = (int64_t)nblk * kGridBlockWords;
-    hipLaunchKernelGGL(k_bm_grid_clear, dim3(grid_for(std::max<int64_t>(words, n_inst), 256)), dim3(256), 0, st, words,
-                       g->slots, n_inst, first ? g->res : nullptr);
-    NFX_LAUNCH_CHECK();
+    NFX_CHECK(grid_clear(g->slots, nblk, g->res, first ? n_inst : 0, st));
     first = false;
     a.blocks = g->blocks + g->wave_at[w];
     void* args[] = {&a};
-    if (hipLaunchCooperativeKernel((const void*)k_bm_grid, dim3(nblk), dim3(kT), args, kGridLdsBytes, st) !=
-        hipSuccess) {
-      (void)hipGetLastError();  // refused (nothing ran): the stepwise kernels take this and the later launches
-      grid_note_refusal();
+    bool ran = false;
+    grid_launch(&g->control, (const void*)k_bm_grid, nblk - (g->control.absent && g->tail[w] ? 1 : 0), args, st, &ran);
+    if (!ran) {  // the stepwise kernels take this and the later launches
       runs_until = w;
       break;
     }
   }
   NFX_CHECK_HIP(hipMemcpyAsync(g->h_res, g->res, sizeof(GridResult) * n_inst, hipMemcpyDeviceToHost, st));
   NFX_CHECK_HIP(hipStreamSynchronize(st));
-  for (int i = 0; i < n_inst; ++i)
-    if (h_mode[i] == 0 && g->wave_of[i] >= 0 && g->wave_of[i] < runs_until && g->h_res[i].status == 0) {
+  for (int i = 0; i < n_inst; ++i) {
+    if (h_mode[i] != 0) continue;
+    if (g->wave_of[i] < runs_until && g->h_res[i].status == 0) {
       (*done)[i] = 1;
       iters[i] = g->h_res[i].iters;
     }
+    ++((*done)[i] ? g->control.solved : g->control.declined);
+  }
   return NFX_OK;
 }
 

@@ -23,6 +23,12 @@ void set_error(const std::string& msg);
     }                                                                           \
   } while (0)
 
+#define NFX_CHECK(expr)           \
+  do {                            \
+    const int _rc = (expr);       \
+    if (_rc != NFX_OK) return _rc; \
+  } while (0)
+
 #define NFX_REQUIRE(cond, msg)                                                  \
   do {                                                                          \
     if (!(cond)) {                                                              \

@@ -12,7 +12,7 @@ int el_grid_blocks(int max_blocks, const nfx_elasticity_tg* pc, int n_blocks);
 int el_grid_capacity();
 
 // One inner solve; vec: 8 vectors of n floats. *status as GridResult::status.
-int el_grid_solve(const MinresGrid* g, int nblk, int n, int n_blocks, const int32_t* brp, const int32_t* bci,
+int el_grid_solve(MinresGrid* g, int nblk, int n, int n_blocks, const int32_t* brp, const int32_t* bci,
                   const float* bva, const nfx_elasticity_tg* pc, const float* rhs, float* x, float* vec, double tol,
                   int maxit, int* iters, int* status, hipStream_t st);
 

@@ -36,12 +36,6 @@ struct ElGridArgs {
   GridResult* res;
 };
 
-__global__ __launch_bounds__(256) void k_el_grid_clear(grid_word* slots, GridResult* res) {
-  const int64_t i = blockIdx.x * 256 + threadIdx.x;
-  if (i < kGridSlotWords) slots[i] = 0;
-  if (i == 0) *res = GridResult{0, 0};
-}
-
 __device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
 __global__ __launch_bounds__(kT) void k_el_grid(ElGridArgs a) {
@@ -459,21 +453,16 @@ int el_grid_blocks(int max_blocks, const nfx_elasticity_tg* pc, int n_blocks) {
   return nblk <= max_blocks && cells(nblk) <= kElGridCells && bytes(nblk) <= kGridLdsBytes ? nblk : 0;
 }
 
-int el_grid_solve(const MinresGrid* g, int nblk, int n, int n_blocks, const int32_t* brp, const int32_t* bci,
+int el_grid_solve(MinresGrid* g, int nblk, int n, int n_blocks, const int32_t* brp, const int32_t* bci,
                   const float* bva, const nfx_elasticity_tg* pc, const float* rhs, float* x, float* vec, double tol,
                   int maxit, int* iters, int* status, hipStream_t st) {
   *status = 1;
-  if (grid_refused()) return NFX_OK;
-  hipLaunchKernelGGL(k_el_grid_clear, dim3(grid_for(kGridSlotWords, 256)), dim3(256), 0, st, g->slots, g->res);
-  NFX_LAUNCH_CHECK();
+  NFX_CHECK(grid_clear(g->slots, nblk, g->res, 1, st));
   ElGridArgs a{n, n_blocks, nblk, maxit, kGridLdsBytes, brp, bci, bva, *pc, rhs, x, vec, tol, g->slots, g->res};
   void* args[] = {&a};
-  if (hipLaunchCooperativeKernel((const void*)k_el_grid, dim3(nblk), dim3(kT), args, kGridLdsBytes, st) != hipSuccess) {
-    (void)hipGetLastError();  // refused (nothing ran): the stepwise kernels take it
-    grid_note_refusal();
-    *status = 1;
-    return NFX_OK;
-  }
+  bool ran = false;
+  grid_launch(&g->control, (const void*)k_el_grid, nblk - (g->control.absent ? 1 : 0), args, st, &ran);
+  if (!ran) return NFX_OK;
   NFX_CHECK_HIP(hipMemcpyAsync(g->h_res, g->res, sizeof(GridResult), hipMemcpyDeviceToHost, st));
   NFX_CHECK_HIP(hipStreamSynchronize(st));
   *iters = g->h_res->iters;

@@ -30,6 +30,22 @@ constexpr int kGridThreads = 1024;
 constexpr int kGridRetrySeconds = 10;
 bool grid_refused();
 void grid_note_refusal();
+
+// what a launch (or one system of it) reports
+struct GridResult {
+  int iters;
+  int status;  // 0 solved or out of iterations, 1 not applicable (nothing was done), 2 a wait was given up
+};
+
+// What a solver object allows, and has seen, of resident launches.
+struct GridControl {
+  int64_t launches = -1;               // still allowed (-1: any number)
+  int absent = 0;                      // != 0: the last block is not launched, the others give up their wait for it
+  int64_t solved = 0, declined = 0;    // inner solves that ran so; that were tried so and ran stepwise
+};
+// Launches kernel on nblk blocks of kGridThreads with all their LDS. *ran = false: not launched (refused, or
+// no more allowed) and nothing ran, the stepwise kernels take it.
+void grid_launch(GridControl* c, const void* kernel, int nblk, void** args, hipStream_t st, bool* ran);
 constexpr int kGridMaxBlocks = 256;
 constexpr int kGridCopies = 8;
 constexpr int kGridBlockWords = 2 * kGridCopies * 2;  // 64-bit words of slots per block
@@ -83,6 +99,9 @@ __device__ __forceinline__ float lanes_total(float v) {
   if (LANES >= 16) v += dpp_move<0x140>(v);  // mirrored in 16: the other eight
   return v;
 }
+
+// Clears the slots of a launch of nblk blocks, and n_res results.
+int grid_clear(grid_word* slots, int nblk, GridResult* res, int n_res, hipStream_t st);
 
 struct GridSync {
   grid_word* slots;   // kGridBlockWords a block, zero before the launch
@@ -159,12 +178,6 @@ __device__ __forceinline__ bool grid_wait(GridSync& g, double& sum) {
   }
   return ok;
 }
-
-// what a launch (or one system of it) reports
-struct GridResult {
-  int iters;
-  int status;  // 0 solved or out of iterations, 1 not applicable (nothing was done), 2 a wait was given up
-};
 
 // The columns that a block's rows meet, as a list, and the rows' columns as 16-bit places in it.
 // Row i has entries start(i) .. start(i) + rowp[i + 1] - rowp[i] of ci; n columns in all.

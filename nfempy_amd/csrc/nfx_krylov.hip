@@ -614,6 +614,29 @@ extern "C" int nfx_solver_destroy(nfx_solver* s) {
   return NFX_OK;
 }
 
+static int resident_set(GridControl* c, int64_t launches, int absent) {
+  NFX_REQUIRE(launches >= -1, "set_resident: launches");
+  c->launches = launches;
+  c->absent = absent;
+  return NFX_OK;
+}
+
+static int resident_counts(const GridControl& c, int64_t* h_counts) {
+  h_counts[0] = c.solved;
+  h_counts[1] = c.declined;
+  return NFX_OK;
+}
+
+extern "C" int nfx_solver_set_resident(nfx_solver* s, int64_t launches, int absent) {
+  NFX_REQUIRE(s, "nfx_solver_set_resident: null pointer");
+  return resident_set(&s->grid.control, launches, absent);
+}
+
+extern "C" int nfx_solver_resident_counts(const nfx_solver* s, int64_t* h_counts) {
+  NFX_REQUIRE(s && h_counts, "nfx_solver_resident_counts: null pointer");
+  return resident_counts(s->grid.control, h_counts);
+}
+
 static int launch_a(nfx_solver* s, const int32_t* rp, const int32_t* ci, const float* va,
                     const float* sign, const float* z, const float* zprev, const float* r1,
                     float* y, float* x, float* wnew, const float* wa, const float* wb, int first,
@@ -757,6 +780,7 @@ extern "C" int nfx_solve_minres_ir(nfx_solver* s, const int32_t* d_rowptr, const
       rc = minres_grid_solve(&s->grid, grid_blocks, s->lanes, n, d_rowptr, d_col, d_val32, d_sign, d_pc_rowptr,
                              d_pc_col, d_pc_val, rf, dx, s->buf, inner_rtol, max_inner, &it, &status, s->stream);
       if (rc) return rc;
+      ++(status ? s->grid.control.declined : s->grid.control.solved);
       if (status) grid_blocks = 0;
     }
     if (!grid_blocks) {
@@ -883,6 +907,7 @@ extern "C" int nfx_solve_minres_ir_tg(nfx_solver* s, const int32_t* d_rowptr, co
       rc = el_grid_solve(&s->grid, grid_blocks, n, s->b3_nblk, s->b3_rp, s->b3_ci, s->b3_va, pc, rf, dx, s->buf,
                          inner_rtol, max_inner, &it, &status, s->stream);
       if (rc) return rc;
+      ++(status ? s->grid.control.declined : s->grid.control.solved);
       if (status) grid_blocks = 0;
     }
     if (!grid_blocks) {
@@ -1338,6 +1363,16 @@ static int bm_set_active(nfx_minres_batch* s, int limit) {
 extern "C" int nfx_minres_batch_destroy(nfx_minres_batch* s) {
   bm_free(s);
   return NFX_OK;
+}
+
+extern "C" int nfx_minres_batch_set_resident(nfx_minres_batch* s, int64_t launches, int absent) {
+  NFX_REQUIRE(s, "nfx_minres_batch_set_resident: null pointer");
+  return resident_set(&s->grid.control, launches, absent);
+}
+
+extern "C" int nfx_minres_batch_resident_counts(const nfx_minres_batch* s, int64_t* h_counts) {
+  NFX_REQUIRE(s && h_counts, "nfx_minres_batch_resident_counts: null pointer");
+  return resident_counts(s->grid.control, h_counts);
 }
 
 extern "C" int64_t nfx_minres_batch_rows(const nfx_minres_batch* s) { return s ? s->n_total : -1; }

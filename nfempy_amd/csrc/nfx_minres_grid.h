@@ -12,6 +12,7 @@ struct MinresGrid {
   grid_word* slots = nullptr;
   GridResult* res = nullptr;
   GridResult* h_res = nullptr;  // pinned
+  GridControl control;
 };
 
 int minres_grid_capacity();

@@ -31,10 +31,10 @@ struct MinresGridArgs {
   GridResult* res;
 };
 
-__global__ __launch_bounds__(256) void k_grid_clear(grid_word* slots, GridResult* res) {
+__global__ __launch_bounds__(256) void k_grid_clear(int64_t words, grid_word* slots, int n_res, GridResult* res) {
   const int64_t i = blockIdx.x * 256 + threadIdx.x;
-  if (i < kGridSlotWords) slots[i] = 0;
-  if (i == 0) *res = GridResult{0, 0};
+  if (i < words) slots[i] = 0;
+  if (i < n_res) res[i] = GridResult{0, 0};
 }
 
 // first row whose weight (6 bytes an entry, 40 a row) reaches b / nblk of the whole
@@ -221,6 +221,26 @@ void grid_note_refusal() {
   g_retry_at.store(grid_clock() + (int64_t)kGridRetrySeconds * 1000000000, std::memory_order_relaxed);
 }
 
+int grid_clear(grid_word* slots, int nblk, GridResult* res, int n_res, hipStream_t st) {
+  const int64_t words = (int64_t)nblk * kGridBlockWords;
+  hipLaunchKernelGGL(k_grid_clear, dim3(grid_for(std::max<int64_t>(words, n_res), 256)), dim3(256), 0, st, words, slots,
+                     n_res, res);
+  NFX_LAUNCH_CHECK();
+  return NFX_OK;
+}
+
+void grid_launch(GridControl* c, const void* kernel, int nblk, void** args, hipStream_t st, bool* ran) {
+  *ran = false;
+  if (c->launches == 0 || grid_refused()) return;
+  if (c->launches > 0) --c->launches;
+  if (hipLaunchCooperativeKernel(kernel, dim3(nblk), dim3(kGridThreads), args, kGridLdsBytes, st) != hipSuccess) {
+    (void)hipGetLastError();
+    grid_note_refusal();
+    return;
+  }
+  *ran = true;
+}
+
 // Resident blocks that the device allows (0: no cooperative launch, or too little LDS).
 int minres_grid_capacity() {
   int dev = 0, coop = 0, cus = 0, per_cu = 0;
@@ -265,20 +285,15 @@ int minres_grid_solve(MinresGrid* g, int nblk, int lanes, int n, const int32_t* 
                       float* x, float* z, double tol, int maxit, int* iters, int* status, hipStream_t st) {
   NFX_REQUIRE(nblk > 0 && nblk <= g->max_blocks, "minres_grid_solve: blocks");
   *status = 1;
-  if (grid_refused()) return NFX_OK;
-  hipLaunchKernelGGL(k_grid_clear, dim3(grid_for(kGridSlotWords, 256)), dim3(256), 0, st, g->slots, g->res);
-  NFX_LAUNCH_CHECK();
+  NFX_CHECK(grid_clear(g->slots, nblk, g->res, 1, st));
   MinresGridArgs a{n, nblk, maxit, kGridLdsBytes, rp, ci, va, sign, prp, pci, pva, rhs, x, z, tol, g->slots, g->res};
   void* args[] = {&a};
   const void* f = lanes == 16  ? (const void*)k_minres_grid<16>
                   : lanes == 8 ? (const void*)k_minres_grid<8>
                                : (const void*)k_minres_grid<4>;
-  if (hipLaunchCooperativeKernel(f, dim3(nblk), dim3(kGridThreads), args, kGridLdsBytes, st) != hipSuccess) {
-    (void)hipGetLastError();  // refused (nothing ran): the stepwise kernels take it
-    grid_note_refusal();
-    *status = 1;
-    return NFX_OK;
-  }
+  bool ran = false;
+  grid_launch(&g->control, f, nblk - (g->control.absent ? 1 : 0), args, st, &ran);
+  if (!ran) return NFX_OK;
   NFX_CHECK_HIP(hipMemcpyAsync(g->h_res, g->res, sizeof(GridResult), hipMemcpyDeviceToHost, st));
   NFX_CHECK_HIP(hipStreamSynchronize(st));
   *iters = g->h_res->iters;

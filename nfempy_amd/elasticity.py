@@ -714,6 +714,7 @@ class ElasticitySystem:
         t1 = time.perf_counter()
         x, info = solver.solve(-self.rhs64, rtol=rtol, inner_rtol=inner_rtol, max_inner=max_inner,
                                max_outer=max_outer)
+        self.last_resident = solver.resident_counts()
         solver.close()
         info["pc"] = pc_kind
         # wall time of the preconditioner set-up (values, blocks, coarse inverse) and of the

@@ -58,6 +58,17 @@ class MinresIR:
             nb, brp, bcol, bval = block3
             nat.call("nfx_solver_set_block3", h, int(nb), nat.ptr(brp), nat.ptr(bcol), nat.ptr(bval))
 
+    def set_resident(self, launches=-1, absent=False):
+        """Resident launches that the solver may still make (-1: any number, 0: stepwise kernels only);
+        ``absent`` makes each of them one that its blocks give up (``nfx_solver_set_resident``)."""
+        nat.call("nfx_solver_set_resident", self._h, launches, int(absent))
+
+    def resident_counts(self):
+        """Inner solves that ran as one resident launch, and those that were tried so and ran stepwise."""
+        out = (ctypes.c_int64 * 2)()
+        nat.call("nfx_solver_resident_counts", self._h, out)
+        return out[0], out[1]
+
     def close(self):
         if getattr(self, "_h", None) is not None and self._h.value:
             nat.lib().nfx_solver_destroy(self._h)
@@ -136,6 +147,17 @@ class MinresBatch:
         self._pc = groups
         n = 0 if groups is None else len(groups)
         nat.call("nfx_minres_batch_set_pc", self._h, n, groups if n else None)
+
+    def set_resident(self, launches=-1, absent=False):
+        """Resident launches that the solver may still make (-1: any number, 0: stepwise kernels only);
+        ``absent`` makes each of them one that its blocks give up (``nfx_minres_batch_set_resident``)."""
+        nat.call("nfx_minres_batch_set_resident", self._h, launches, int(absent))
+
+    def resident_counts(self):
+        """Inner solves of instances that ran as one resident launch, and those that were tried so and ran stepwise."""
+        out = (ctypes.c_int64 * 2)()
+        nat.call("nfx_minres_batch_resident_counts", self._h, out)
+        return out[0], out[1]
 
     def close(self):
         if getattr(self, "_h", None) is not None and self._h.value:

@@ -69,6 +69,8 @@ def test_resident_route_matches_stepwise(n, kind):
             x = x.cpu().numpy()
             assert info["converged"], (name, info)
             assert np.linalg.norm(b - A @ x) <= 1.1 * RTOL * np.linalg.norm(b), name
+        solved, declined = s.resident_counts()
+        assert (solved > 0 and declined == 0) if name == "resident" else solved == 0, (name, solved, declined)
         got[name] = info["iterations"], x
         s.close()
     # the same recurrence, tested every 16 iterations: roundings can move a stop by one test per outer step
@@ -126,7 +128,9 @@ def test_batch_over_resident_sizes(pc):
     b.assemble()
     print(f"[minres grid] batch {pc}", flush=True)
     mixed, mixed_infos, _ = b.solve_batched(rtol=1e-8, pc=pc)
+    assert (b.last_resident[0] > 0) == (pc == "diag")  # the limit is one of the cycle's
     xs, infos, _ = b.solve_batched(list(range(7)), rtol=1e-8, pc=pc)
+    assert b.last_resident[0] == sum(i["outer"] for i in infos) and b.last_resident[1] == 0
     xs.append(mixed[7])
     infos.append(mixed_infos[7])
     for i in range(7):  # both within rtol of the solution, times the conditioning
@@ -141,6 +145,7 @@ def test_batch_over_resident_sizes(pc):
         assert res <= 1.1e-8, (i, res)
     for i in (1, 2, 3, 6):
         alone, info, _ = b.solve_batched([i], rtol=1e-8, pc=pc)
+        assert b.last_resident == (info[0]["outer"], 0)
         assert info[0]["iterations"] == infos[i]["iterations"]
         assert torch.equal(alone[0], xs[i]), i
 
@@ -173,6 +178,7 @@ def test_elasticity_resident_matches_stepwise(n):
         print(f"[minres grid] elasticity n={n} blocks={block3}", flush=True)
         x, info = y.solve(rtol=1e-9)
         assert info["converged"] and info["residual"] <= 1e-9, info
+        assert y.last_resident == ((info["outer"], 0) if block3 else (0, 0)), (n, y.last_resident)
         rp, col, _, v64 = y.full("A")
         A = torch.sparse_csr_tensor(rp.long(), col.long(), v64, size=(y.n, y.n))
         res = float((-y.rhs64 - A @ x).norm() / y.rhs64.norm())

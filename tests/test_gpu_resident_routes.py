@@ -110,3 +110,244 @@ def test_incomplete_preconditioners_are_refused():
     x, info = s.solve(-y.rhs64, rtol=1e-8)
     assert info["converged"]
     s.close()
+
+
+# ---- which route ran ------------------------------------------------------------------------------
+LDS = 158 * 1024  # bytes of a block, as nfx_grid.h has them
+SHARE = 128 * 1024  # bytes of an instance per block, as nfx_bm_grid.hip has them
+
+
+def _batch_layout(A):
+    """(values in LDS, columns beyond what the threads hold) of each block of an instance without a two-grid cycle: how
+    nfx_bm_grid.hip lays out its LDS."""
+    n = A.shape[0]
+    blocks = -(-(6 * A.nnz + 40 * n) // SHARE)
+    out = set()
+    for r in range(blocks):
+        S = A[n * r // blocks:n * (r + 1) // blocks]
+        R, H = S.shape[0], len(np.unique(S.indices))
+        base = 4 * (2 * R + 1) + 24 * R + 4 + 4 * ((S.nnz + 1) // 2)
+        assert base + 8 * ((n + 31) // 32) + 4 * H <= LDS and base + 8 * H <= LDS
+        listed = H > 4 * 1024
+        out.add((base + (8 if listed else 4) * H + 4 * S.nnz <= LDS, listed))
+    return out
+
+
+@pytest.mark.parametrize("n,kind,layout", [(8000, 1, (True, False)), (8000, 2, (True, True)),
+                                           (20000, 9, (False, True))])
+def test_batch_layouts_match_stepwise(n, kind, layout):
+    """Scattered systems whose blocks meet few or many columns, and hold their values in LDS or not: the resident
+    route against the stepwise one and the FP64 residual."""
+    import torch
+
+    from nfempy_amd.solvers import MinresBatch
+    from tests.test_gpu_minres_grid import _matrix
+
+    print(f"[routes] layout n={n} {kind}", flush=True)
+    A, d = _matrix(n, kind, seed=n + kind)
+    A.sort_indices()
+    assert layout in _batch_layout(A)
+    dev = lambda a, t: torch.tensor(np.ascontiguousarray(a), dtype=t, device="cuda")
+    v64 = dev(A.data, torch.float64)
+    b = np.random.default_rng(n).standard_normal(n)
+    got = {}
+    for launches in (-1, 0):
+        mb = MinresBatch([{"rowptr": dev(A.indptr, torch.int32), "col": dev(A.indices, torch.int32),
+                           "vals32": v64.to(torch.float32), "vals64": v64, "pinv": dev(1.0 / d, torch.float32)}])
+        mb.set_resident(launches)
+        x, infos = mb.solve(dev(b, torch.float64), rtol=1e-9)
+        x = x.cpu().numpy()
+        assert infos[0]["converged"]
+        assert mb.resident_counts() == ((infos[0]["outer"], 0) if launches else (0, 0))
+        assert np.linalg.norm(b - A @ x) <= 1.1e-9 * np.linalg.norm(b)
+        got[launches] = x
+        mb.close()
+    # eigenvalues of at least 1 in magnitude: an error is at most the residual, 1e-9 |b| for each route
+    assert np.linalg.norm(got[-1] - got[0]) <= 2.2e-9 * np.linalg.norm(b)
+
+
+def _elasticity_layout(bp, bc, mem, E, ns, n_agg):
+    """(values in LDS, columns beyond what the threads hold) of the blocks of an elasticity solve on the 3 x 3
+    block rows (bp, bc): nfx_el_grid.hip's layout."""
+    nb, nu = len(bp) - 1, 3 * E
+    F, n = ns // 9, 3 * nb
+    size = lambda k: (2 * int(bp[-1]) + 64 * n) // k + (48 << 10)
+    blocks = 16
+    while blocks < 256 and (-(-E // blocks) > 12 or size(blocks) > LDS):
+        blocks *= 2
+    assert -(-E // blocks) <= 34 and size(blocks) <= LDS and n_agg <= 128
+    out = set()
+    for k in range(blocks):
+        f = np.arange(3 * (F * k // blocks), 3 * (F * (k + 1) // blocks))
+        c = mem[E * k // blocks:E * (k + 1) // blocks]
+        rows = np.concatenate([f, ns // 3 + c, (ns + nu) // 3 + c])
+        RB, nz = len(rows), int((bp[rows + 1] - bp[rows]).sum())
+        H = len(np.unique(np.concatenate([bc[bp[r]:bp[r + 1]] for r in rows])))
+        words = 2 * RB + 1 + 15 * RB + 27 * len(f) + 3 * 1024 + 6 * 384 + 12 * 128 + 384 + 129 + 256
+        base = 4 * words + 4 * ((nz + 1) // 2)
+        assert base + 8 * ((nb + 31) // 32) + 4 * H <= LDS and base + 16 * H <= LDS
+        listed = 3 * H > 4 * 1024
+        out.add((base + 12 * H + (4 * H if listed else 0) + 36 * nz <= LDS, listed))
+    return out
+
+
+@pytest.mark.parametrize("n,shuffled,layout", [(5, False, (True, False)), (10, False, (False, False)),
+                                               (10, True, (False, True))])
+def test_elasticity_layouts_are_resident(n, shuffled, layout):
+    """Systems whose blocks hold their values in LDS, and the largest that is resident, whose blocks do not;
+    with its faces numbered in any order a block meets more columns than its threads hold. FP64 residuals."""
+    import scipy.sparse as sps
+    import torch
+
+    from nfempy_amd.solvers import MinresIR
+
+    print(f"[routes] elasticity layout n={n} {shuffled}", flush=True)
+    y = _elasticity(n)
+    desc = _copy(y.twogrid().setup())
+    rp, col, v32, v64 = (v.cpu().numpy() for v in y.full("A"))
+    A = sps.csr_matrix((v64, col, rp), shape=(y.n, y.n))
+    F = y.n_s // 9
+    p = np.random.default_rng(n).permutation(F) if shuffled else np.arange(F)
+    rows = np.concatenate([(9 * p[:, None] + np.arange(9)).ravel(), np.arange(y.n_s, y.n)])
+    A = A[rows][:, rows].tocsr()
+    A.sort_indices()
+    B = A.tobsr((3, 3))
+    B.sort_indices()
+    mem = y.twogrid().agg_mem.cpu().numpy()
+    seen = _elasticity_layout(B.indptr, B.indices, mem, y.E, y.n_s, desc.n_agg)
+    print(f"[routes] {seen}", flush=True)
+    assert layout in seen
+    dev = lambda a, t: torch.tensor(np.ascontiguousarray(a), dtype=t, device="cuda")
+    i32, f32, f64 = torch.int32, torch.float32, torch.float64
+    dinv = y.twogrid().dinv32.view(F, 81)[torch.tensor(p, device="cuda")].contiguous()
+    desc.dinv = dinv.data_ptr()
+    block3 = (len(B.indices), dev(B.indptr, i32), dev(B.indices, i32),
+              dev(B.data.reshape(-1, 9).T.ravel(), f32))
+    s = MinresIR(dev(A.indptr, i32), dev(A.indices, i32), dev(A.data, f32), dev(A.data, f64), block3=block3, tg=desc)
+    b = -y.rhs64.cpu().numpy()[rows]
+    x, info = s.solve(dev(b, f64), rtol=1e-8, inner_rtol=3e-4)
+    assert info["converged"] and s.resident_counts() == (info["outer"], 0)
+    s.close()
+    assert np.linalg.norm(b - A @ x.cpu().numpy()) <= 1.1e-8 * np.linalg.norm(b)
+
+
+def _single(n=4000, stream=None):
+    import torch
+
+    from nfempy_amd.solvers import MinresIR
+    from tests.test_gpu_minres_grid import _matrix
+
+    A, d = _matrix(n, 6, seed=n)
+    A.sort_indices()
+    dev = lambda a, t: torch.tensor(np.ascontiguousarray(a), dtype=t, device="cuda")
+    v64 = dev(A.data, torch.float64)
+    s = MinresIR(dev(A.indptr, torch.int32), dev(A.indices, torch.int32), v64.to(torch.float32), v64,
+                 pinv=dev(1.0 / d, torch.float32), stream=stream)
+    return s, dev(np.random.default_rng(n).standard_normal(n), torch.float64)
+
+
+def test_stepwise_where_no_launch_is_allowed():
+    """None, one, and as many launches as a solve wants: the counts say what ran, every solve converges."""
+    print("[routes] single", flush=True)
+    s, b = _single()
+    full, info = s.solve(b, rtol=1e-10)
+    outer = info["outer"]
+    assert outer > 1 and s.resident_counts() == (outer, 0)
+    s.set_resident(0)
+    x, info = s.solve(b, rtol=1e-10)
+    assert info["converged"] and s.resident_counts() == (outer, 1)
+    s.set_resident(1)  # the second inner solve is declined
+    x, info = s.solve(b, rtol=1e-10)
+    assert info["converged"] and s.resident_counts() == (outer + 1, 2)
+    s.set_resident()
+    x, info = s.solve(b, rtol=1e-10)
+    assert s.resident_counts() == (2 * outer + 1, 2) and bool((x == full).all())
+    s.close()
+
+    print("[routes] elasticity", flush=True)
+    y = _elasticity(3)
+    s, _ = _elasticity_solver(y)
+    s.set_resident(1)
+    x, info = s.solve(-y.rhs64, rtol=1e-9, inner_rtol=3e-4)
+    assert info["converged"] and info["outer"] > 1 and s.resident_counts() == (1, 1)
+    s.close()
+
+    print("[routes] batch over two launches", flush=True)
+    _, mb, rhs, _ = _batch([(9, 2), (5, 2), (9, 2), (9, 2), (3, 1)])
+    mb.set_resident(1)
+    x, infos = mb.solve(rhs, rtol=1e-8)
+    solved, declined = mb.resident_counts()
+    assert all(i["converged"] for i in infos) and 0 < solved < 5 and declined > 0
+    mb.close()
+
+
+def test_given_up_waits_end_stepwise():
+    """A launch without its last block: the others give up their wait for it, the launch ends, the solve goes on
+    with the stepwise kernels."""
+    print("[routes] single", flush=True)
+    s, b = _single()
+    s.set_resident(absent=True)
+    x, info = s.solve(b, rtol=1e-9)
+    assert info["converged"] and s.resident_counts() == (0, 1)
+    s.set_resident()
+    x, info = s.solve(b, rtol=1e-9)
+    assert s.resident_counts() == (info["outer"], 1)
+    s.close()
+
+    print("[routes] elasticity", flush=True)
+    y = _elasticity(3)
+    s, _ = _elasticity_solver(y)
+    s.set_resident(absent=True)
+    x, info = s.solve(-y.rhs64, rtol=1e-8)
+    assert info["converged"] and s.resident_counts() == (0, 1)
+    s.close()
+
+    print("[routes] batch", flush=True)
+    _, mb, rhs, _ = _batch([(7, 2), (6, 2)])
+    mb.set_resident(absent=True)
+    x, infos = mb.solve(rhs, rtol=1e-8)
+    solved, declined = mb.resident_counts()
+    assert all(i["converged"] for i in infos) and declined >= 1
+    mb.close()
+
+
+def test_two_threads_on_two_streams():
+    """Two host threads, each with its own solver and stream: every answer is the one that the solver gives
+    alone (bitwise, as long as no launch was declined)."""
+    import threading
+
+    import torch
+
+    print("[routes] two threads", flush=True)
+    pair, want, got = [], [], [[], []]
+    for n in (4000, 9001):
+        st = torch.cuda.Stream()
+        with torch.cuda.stream(st):
+            s, b = _single(n, stream=st)
+            want.append(s.solve(b, rtol=1e-9)[0])
+        pair.append((s, b, st))
+    torch.cuda.synchronize()
+
+    def work(i):
+        s, b, st = pair[i]
+        with torch.cuda.stream(st):
+            for _ in range(8):
+                got[i].append(s.solve(b, rtol=1e-9))
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for th in threads:
+        th.start()
+    for th in threads:
+        th.join()
+    torch.cuda.synchronize()
+    for i, (s, b, _) in enumerate(pair):
+        assert len(got[i]) == 8 and all(info["converged"] for _, info in got[i])
+        solved, declined = s.resident_counts()
+        print(f"[routes] solver {i}: {solved} resident, {declined} declined", flush=True)
+        assert solved > 0
+        for x, _ in got[i]:
+            if declined == 0:
+                assert torch.equal(x, want[i])
+            else:
+                assert float((x - want[i]).norm()) <= 2.2e-9 * float(b.norm())
+        s.close()
