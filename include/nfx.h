@@ -438,7 +438,10 @@ int nfx_solve_minres_ir_tg(nfx_solver* s, const int32_t* d_rowptr, const int32_t
  * (FP32 inverse diagonal, NULL = identity), its own MINRES recurrence, stopping test and FP64
  * refinement to ||b - A x|| / ||b|| <= rtol; vectors are concatenated in instance order
  * (row_off is filled in by nfx_minres_batch_create). Partial sums are reduced per instance in
- * a fixed order: results do not depend on the other instances of the batch. */
+ * a fixed order: on one route (resident or stepwise, nfx_minres_batch_set_resident) an instance's
+ * result is bitwise the same whatever the other instances are. The route of a solve is that of the
+ * whole batch, chosen before its first iteration from the sizes of all instances: between routes
+ * results differ by roundings (both end at rtol). */
 typedef struct nfx_minres_batch_item {
   int n_rows;
   int lanes; /* filled in by nfx_minres_batch_create (lanes per row of the SpMV) */

@@ -14,7 +14,7 @@ struct BmGridBlock {
 };
 
 // Launch plan and work space of a batch. An instance's block count follows from its own size, so its
-// sums, and its result, are the same in every batch that is resident.
+// sums, and its result, are the same in every batch that is resident; a stepwise batch has other roundings.
 struct BmGrid {
   char *dev = nullptr, *host = nullptr;  // one allocation each
   std::vector<int> wave_of;    // launch of each instance, -1: not resident
@@ -38,8 +38,12 @@ int bm_grid_create(BmGrid* g, int n_inst, const nfx_minres_batch_item* items, co
                    hipStream_t st);
 void bm_grid_destroy(BmGrid* g);
 
-// Inner solves of the resident instances with h_mode 0. done[i]: set where instance i was solved, with
-// iters[i] and its rows of x. vec: 8 vectors of n_total floats, own: 3 more.
+// The route of a whole solve, from all instances of the batch, whichever still iterate: resident or not.
+int bm_grid_route(BmGrid* g, int n_inst, int64_t n_total, const std::vector<nfx_batch_tg>& pc, bool* resident,
+                  hipStream_t st);
+
+// Inner solves of the instances with h_mode 0 on the resident route. done[i]: set where instance i was solved,
+// with iters[i] and its rows of x. vec: 8 vectors of n_total floats, own: 3 more.
 int bm_grid_solve(BmGrid* g, int n_inst, int64_t n_total, const nfx_minres_batch_item* d_items, const int32_t* d_mode,
                   const int32_t* h_mode, const std::vector<nfx_batch_tg>& pc, const float* rhs, float* x, float* vec,
                   float* own, const double* tol, int maxit, int* iters, std::vector<char>* done, hipStream_t st);

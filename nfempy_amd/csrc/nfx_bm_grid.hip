@@ -628,26 +628,46 @@ void bm_grid_destroy(BmGrid* g) {
   *g = BmGrid();
 }
 
+int bm_grid_route(BmGrid* g, int n_inst, int64_t n_total, const std::vector<nfx_batch_tg>& pc, bool* resident,
+                  hipStream_t st) {
+  *resident = false;
+  if (n_total > INT32_MAX || !g->control.launches || grid_refused()) return NFX_OK;
+  // all or none: beside instances that have to iterate stepwise the others cost little there and a launch
+  // each here (32 instances up to 16 x 16 x 16 cubes: 79.5 ms stepwise, 94.5 ms split)
+  for (int i = 0; i < n_inst; ++i)
+    if (g->wave_of[i] < 0) return NFX_OK;
+  hipLaunchKernelGGL(k_bm_grid_zero, dim3(grid_for(n_inst * kBmRanges, 256)), dim3(256), 0, st, n_inst * kBmRanges,
+                     g->ranges);
+  for (size_t q = 0; q < pc.size(); ++q) {
+    hipLaunchKernelGGL(k_bm_ranges, dim3(grid_for(pc[q].n_cells, 256)), dim3(256), 0, st, pc[q].n_cells,
+                       pc[q].cell_inst, n_inst, (int)q, 0, pc[q].agg_of, pc[q].alen, g->ranges);
+    if (pc[q].n_fb > 0)
+      hipLaunchKernelGGL(k_bm_ranges, dim3(grid_for(pc[q].n_fb, 256)), dim3(256), 0, st, pc[q].n_fb, pc[q].fb_inst,
+                         n_inst, (int)q, 1, nullptr, nullptr, g->ranges);
+  }
+  NFX_LAUNCH_CHECK();
+  if (!pc.empty()) {
+    std::vector<int32_t> r((size_t)n_inst * kBmRanges);
+    NFX_CHECK_HIP(hipMemcpyAsync(r.data(), g->ranges, sizeof(int32_t) * r.size(), hipMemcpyDeviceToHost, st));
+    NFX_CHECK_HIP(hipStreamSynchronize(st));
+    for (int i = 0; i < n_inst; ++i)
+      if (r[(size_t)i * kBmRanges + 12] > kBmGridAgg) return NFX_OK;
+  }
+  *resident = true;
+  return NFX_OK;
+}
+
 int bm_grid_solve(BmGrid* g, int n_inst, int64_t n_total, const nfx_minres_batch_item* d_items, const int32_t* d_mode,
                   const int32_t* h_mode, const std::vector<nfx_batch_tg>& pc, const float* rhs, float* x, float* vec,
                   float* own, const double* tol, int maxit, int* iters, std::vector<char>* done, hipStream_t st) {
   done->assign(n_inst, 0);
   const int waves = (int)g->wave_at.size() - 1;
-  std::vector<char> runs(std::max(waves, 1), 0);
-  bool any = false;
-  // all or none: beside instances that have to iterate stepwise the others cost little there and a launch
-  // each here (32 instances up to 16 x 16 x 16 cubes: 79.5 ms stepwise, 94.5 ms split)
-  for (int i = 0; i < n_inst; ++i)
-    if (h_mode[i] == 0) {
-      if (g->wave_of[i] < 0) return NFX_OK;
-      any = runs[g->wave_of[i]] = 1;
-    }
-  if (!any || n_total > INT32_MAX || !g->control.launches || grid_refused()) return NFX_OK;
-
-  for (int i = 0; i < n_inst; ++i) g->h_tol[i] = tol[i];
+  std::vector<char> runs(waves, 0);
+  for (int i = 0; i < n_inst; ++i) {
+    if (h_mode[i] == 0) runs[g->wave_of[i]] = 1;
+    g->h_tol[i] = tol[i];
+  }
   NFX_CHECK_HIP(hipMemcpyAsync(g->tol, g->h_tol, sizeof(double) * n_inst, hipMemcpyHostToDevice, st));
-  hipLaunchKernelGGL(k_bm_grid_zero, dim3(grid_for(n_inst * kBmRanges, 256)), dim3(256), 0, st, n_inst * kBmRanges,
-                     g->ranges);
   BmGridArgs a{};
   a.items = d_items;
   a.mode = d_mode;
@@ -663,23 +683,7 @@ int bm_grid_solve(BmGrid* g, int n_inst, int64_t n_total, const nfx_minres_batch
   a.tol = g->tol;
   a.slots = g->slots;
   a.res = g->res;
-  for (int q = 0; q < a.n_groups; ++q) {
-    a.pc[q] = pc[q];
-    hipLaunchKernelGGL(k_bm_ranges, dim3(grid_for(pc[q].n_cells, 256)), dim3(256), 0, st, pc[q].n_cells,
-                       pc[q].cell_inst, n_inst, q, 0, pc[q].agg_of, pc[q].alen, g->ranges);
-    if (pc[q].n_fb > 0)
-      hipLaunchKernelGGL(k_bm_ranges, dim3(grid_for(pc[q].n_fb, 256)), dim3(256), 0, st, pc[q].n_fb, pc[q].fb_inst,
-                         n_inst, q, 1, nullptr, nullptr, g->ranges);
-  }
-  NFX_LAUNCH_CHECK();
-  if (a.n_groups) {
-    // an instance with too many aggregates for the cycle here: the batch stays together
-    std::vector<int32_t> r((size_t)n_inst * kBmRanges);
-    NFX_CHECK_HIP(hipMemcpyAsync(r.data(), g->ranges, sizeof(int32_t) * r.size(), hipMemcpyDeviceToHost, st));
-    NFX_CHECK_HIP(hipStreamSynchronize(st));
-    for (int i = 0; i < n_inst; ++i)
-      if (h_mode[i] == 0 && r[(size_t)i * kBmRanges + 12] > kBmGridAgg) return NFX_OK;
-  }
+  for (int q = 0; q < a.n_groups; ++q) a.pc[q] = pc[q];
   bool first = true;
   int runs_until = waves;
   for (int w = 0; w < waves; ++w) {

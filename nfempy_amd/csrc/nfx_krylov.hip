@@ -1504,6 +1504,8 @@ extern "C" int nfx_solve_minres_batch_ir(nfx_minres_batch* s, const double* d_b,
     h_outer[i] = 0;
     h_resid[i] = 0;
   }
+  bool resident = false;  // the route, chosen before the first inner solve
+  bool routed = false;
   for (int outer = 0; outer <= max_outer; ++outer) {
     int n_act = 0;
     for (int i = 0; i < m; ++i) {
@@ -1553,26 +1555,32 @@ extern "C" int nfx_solve_minres_batch_ir(nfx_minres_batch* s, const double* d_b,
     NFX_LAUNCH_CHECK();
     // the inner solve changes h_mode: keep the outer set for the update that follows
     std::vector<int32_t> mode_outer(s->h_mode, s->h_mode + m);
-    // instances that fit a few CUs as resident launches, the rest stepwise together
-    std::vector<char> done;
-    std::vector<int> resident(m, 0);
-    rc = nfx::batch_tg_check(s->pc.data(), (int)s->pc.size());
-    if (rc) return rc;
-    rc = nfx::bm_grid_solve(&s->grid, m, N, s->items, s->mode, s->h_mode, s->pc, rf, dx, s->buf, s->buf + N * 10, tol.data(),
-                            max_inner, resident.data(), &done, st);
-    if (rc) return rc;
-    bool rest = false;
-    for (int i = 0; i < m; ++i) {
-      if (done[i]) s->h_mode[i] = 2;
-      rest = rest || s->h_mode[i] == 0;
+    if (!routed) {
+      rc = nfx::batch_tg_check(s->pc.data(), (int)s->pc.size());
+      if (rc) return rc;
+      rc = nfx::bm_grid_route(&s->grid, m, N, s->pc, &resident, st);
+      if (rc) return rc;
+      routed = true;
     }
     std::fill(it.begin(), it.end(), 0);
+    std::vector<int> stepwise(m, 0);
+    bool rest = !resident;
+    if (resident) {
+      std::vector<char> done;
+      rc = nfx::bm_grid_solve(&s->grid, m, N, s->items, s->mode, s->h_mode, s->pc, rf, dx, s->buf, s->buf + N * 10,
+                              tol.data(), max_inner, it.data(), &done, st);
+      if (rc) return rc;
+      for (int i = 0; i < m; ++i) {
+        if (done[i]) s->h_mode[i] = 2;
+        rest = rest || s->h_mode[i] == 0;
+      }
+    }
     if (rest) {
-      rc = bm_inner(s, rf, dx, tol.data(), max_inner, it.data());
+      rc = bm_inner(s, rf, dx, tol.data(), max_inner, stepwise.data());
       if (rc) return rc;
     }
     for (int i = 0; i < m; ++i) {
-      h_iters[i] += done[i] ? resident[i] : it[i];
+      h_iters[i] += it[i] + stepwise[i];
       s->h_mode[i] = mode_outer[i];
     }
     NFX_CHECK_HIP(hipMemcpyAsync(s->mode, s->h_mode, sizeof(int32_t) * m, hipMemcpyHostToDevice, st));

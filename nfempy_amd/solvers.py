@@ -115,8 +115,9 @@ class MinresIR:
 
 class MinresBatch:
     """Batched FP32 MINRES + FP64 refinement over independent systems (``nfx_minres_batch``):
-    one set of launches per iteration for all instances, each with its own recurrence,
-    stopping test and refinement. ``systems``: dicts with rowptr, col, vals32, vals64 and
+    one set of launches per iteration for all instances (small batches: one launch per inner
+    solve, ``set_resident``), each with its own recurrence, stopping test and refinement; on
+    either route an instance's result does not depend on the other instances. ``systems``: dicts with rowptr, col, vals32, vals64 and
     optional sign / pinv (the symmetric form D A and a diagonal preconditioner)."""
 
     def __init__(self, systems, stream=None):

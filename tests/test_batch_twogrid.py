@@ -12,7 +12,7 @@ GPU: one application on a mixed RT1-P0 / RT2-P1 batch equals the dense cycle
 instances' FP64 matrices (W = omega S_cc^-1 per cell, P the aggregates' indicator), to 1e-4
 relative; the batched MINRES with the cycle reaches 1e-8 against the oracle-assembled
 systems in far fewer iterations than with the diagonal, and an instance's result is bitwise
-the same when it is solved alone.
+the same when it is solved alone (on the same route: these are resident).
 """
 
 import numpy as np

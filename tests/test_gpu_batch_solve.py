@@ -2,7 +2,8 @@
 
 Every instance of a mixed RT1-P0 / RT2-P1 batch reaches an FP64 relative residual of
 1e-8 against the oracle-assembled system (scipy's sparse LU of that system agrees to
-1e-6); an instance's result does not depend on the other instances of the batch
+1e-6); on one route (small batches like these are resident, alone as together) an
+instance's result does not depend on the other instances of the batch
 (bitwise equal when it is solved alone); the per-instance iteration counts stay within a
 check interval of the single-system MINRES's or below (same recurrence, other reduction
 order, refinement steps that stop at the reduction still missing).

@@ -11,22 +11,29 @@ pytestmark = pytest.mark.gpu
 
 def _batch(specs, pc="twogrid", seed=3):
     """(DarcyBatch, MinresBatch, right-hand sides, BatchTwoGrid or None) with the preconditioner set up."""
+    from nfempy_amd.batch import DarcyBatch
+
+    b = DarcyBatch(specs, seed=seed, workers=1)
+    b.assemble()
+    return _batch_of(b, *range(len(specs)), pc=pc)
+
+
+def _batch_of(b, *idx, pc="twogrid"):
+    """The same of some instances of a batch."""
     import torch
 
-    from nfempy_amd.batch import DarcyBatch
     from nfempy_amd.batch_pc import BatchTwoGrid
     from nfempy_amd.learned import default_weights_path, load_params
     from nfempy_amd.solvers import MinresBatch
 
-    b = DarcyBatch(specs, seed=seed, workers=1)
-    b.assemble()
-    systems = [b.fp64_system(i) for i in range(len(specs))]
+    systems = [b.fp64_system(i) for i in idx]
     mb = MinresBatch(systems)
     tg = None
     if pc != "diag":
         theta = load_params(default_weights_path()) if pc == "learned" else None
-        tg = BatchTwoGrid([inst["system"] for inst in b.instances], mb.offsets, theta=theta)
+        tg = BatchTwoGrid([b.instances[i]["system"] for i in idx], mb.offsets, theta=theta)
         mb.set_pc(tg.setup([s["vals64"] for s in systems]))
+        mb._tg = tg  # the descriptors point into its arrays
     return b, mb, torch.cat([s["b"] for s in systems]), tg
 
 
@@ -351,3 +358,31 @@ def test_two_threads_on_two_streams():
             else:
                 assert float((x - want[i]).norm()) <= 2.2e-9 * float(b.norm())
         s.close()
+
+
+def test_a_batch_keeps_one_route():
+    """The route is that of the whole batch, whichever instances still iterate: with an instance that the cycle
+    leaves to the stepwise kernels (11 cubed: 216 aggregates) the others' results are bitwise the same while
+    it iterates, when it starts from its solution, and when the batch is kept from resident launches; alone
+    on the stepwise route each instance is bitwise what it is there."""
+    import torch
+
+    print("[routes] one route", flush=True)
+    specs = [(4, 1), (5, 2), (11, 1), (3, 2)]
+    b, mb, rhs, _ = _batch(specs)
+    x, infos = mb.solve(rhs, rtol=1e-8)
+    assert all(i["converged"] for i in infos) and mb.resident_counts() == (0, 0)
+    part = lambda v, i: v[int(mb.offsets[i]):int(mb.offsets[i + 1])]
+    start = torch.zeros_like(rhs)
+    part(start, 2).copy_(part(x, 2))
+    again, infos2 = mb.solve(rhs, x=start, rtol=1e-8)
+    assert infos2[2]["iterations"] == 0 and mb.resident_counts() == (0, 0)
+    for i in (0, 1, 3):
+        assert torch.equal(part(again, i), part(x, i)), i
+    mb.close()
+    for i in (0, 1, 3):
+        _, one, rhs1, _ = _batch_of(b, i)
+        one.set_resident(0)
+        alone, info = one.solve(rhs1, rtol=1e-8)
+        assert info[0]["iterations"] == infos[i]["iterations"] and torch.equal(alone, part(x, i)), i
+        one.close()
