@@ -17,6 +17,7 @@ struct BmGridBlock {
 // sums, and its result, are the same in every batch that is resident; a stepwise batch has other roundings.
 struct BmGrid {
   char *dev = nullptr, *host = nullptr;  // one allocation each
+  int cap = 0;                 // blocks of a launch
   std::vector<int> wave_of;    // launch of each instance, -1: not resident
   std::vector<int> wave_at;    // first block of each launch in blocks[], and the end
   std::vector<char> tail;      // per launch: its last block is one of several of an instance

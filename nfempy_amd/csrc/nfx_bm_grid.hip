@@ -26,6 +26,16 @@ constexpr int kBmGridAgg = 128;    // coarse unknowns of an instance: 16 inverse
 // Bytes of an instance (6 an entry, 40 a row) per block: what leaves room for the values in LDS. Half of
 // it is no faster (the sums over twice the blocks take longer) and fills two launches instead of one.
 constexpr int64_t kBmGridShare = 128 << 10;
+// Launches of a resident batch: they run one after the other, 10-18 us an iteration each, where the stepwise
+// kernels take all instances in the same launches (25 us an iteration with the diagonal, 56 with the cycle, and
+// 7-15 for what a full launch here holds). Up to three pay, up to six where they are three quarters full. Set-up
+// and solve in ms, resident / stepwise, diagonal | two-grid: instances of 9 cubed of degree 2 (87 blocks, two a
+// launch) in 1 launch 12.6/35.1 | 5.1/15.1, in 2 24.1/39.2 | 9.7/16.5, in 3 35.9/42.4 | 14.6/18.4, in 4 46.4/45.6
+// | 19.2/19.6, in 6 68.5/64.9 | 28.4/25.9, in 12 137/98 | 56/43; of 5 cubed (15 blocks, 17 a launch) in 3
+// 19.7/26.6 | 12.9/17.1, in 6 38.8/43.7 | 25.3/26.7; of degree 1, 6 cubed (3 blocks) in 3 8.0/11.9 | 9.8/13.5.
+inline bool bm_grid_pays(int launches, int blocks, int cap) {
+  return launches <= 3 || (launches <= 6 && 4 * (int64_t)blocks >= 3 * (int64_t)launches * cap);
+}
 
 struct BmGridArgs {
   const nfx_minres_batch_item* items;
@@ -566,7 +576,7 @@ int bm_grid_create(BmGrid* g, int n_inst, const nfx_minres_batch_item* items, co
     (void)hipGetLastError();
     return NFX_OK;
   }
-  const int cap = std::min(cus, kGridMaxBlocks);
+  const int cap = g->cap = std::min(cus, kGridMaxBlocks);
 
   // one device and one pinned allocation
   size_t at = 0;
@@ -636,6 +646,7 @@ int bm_grid_route(BmGrid* g, int n_inst, int64_t n_total, const std::vector<nfx_
   // each here (32 instances up to 16 x 16 x 16 cubes: 79.5 ms stepwise, 94.5 ms split)
   for (int i = 0; i < n_inst; ++i)
     if (g->wave_of[i] < 0) return NFX_OK;
+  if (!bm_grid_pays((int)g->wave_at.size() - 1, g->wave_at.back(), g->cap)) return NFX_OK;
   hipLaunchKernelGGL(k_bm_grid_zero, dim3(grid_for(n_inst * kBmRanges, 256)), dim3(256), 0, st, n_inst * kBmRanges,
                      g->ranges);
   for (size_t q = 0; q < pc.size(); ++q) {

@@ -386,3 +386,15 @@ def test_a_batch_keeps_one_route():
         alone, info = one.solve(rhs1, rtol=1e-8)
         assert info[0]["iterations"] == infos[i]["iterations"] and torch.equal(alone, part(x, i)), i
         one.close()
+
+
+@pytest.mark.parametrize("spec,count,resident", [((9, 2), 6, True), ((9, 2), 7, False), ((5, 2), 96, True)])
+def test_a_batch_is_resident_where_its_launches_pay(spec, count, resident):
+    """Instances of 9 cubed of degree 2 take 87 blocks, two a launch of 256: three launches pay, four, two
+    thirds full, do not. Instances of 5 cubed take 15 blocks: six launches for 1,440 of them pay."""
+    print(f"[routes] launches of {count}", flush=True)
+    b, mb, rhs, _ = _batch([spec] * count)
+    x, infos = mb.solve(rhs, rtol=1e-8)
+    assert all(i["converged"] for i in infos)
+    assert mb.resident_counts() == ((sum(i["outer"] for i in infos), 0) if resident else (0, 0))
+    mb.close()
