@@ -705,7 +705,8 @@ int bm_grid_solve(BmGrid* g, int n_inst, int64_t n_total, const nfx_minres_batch
     a.blocks = g->blocks + g->wave_at[w];
     void* args[] = {&a};
     bool ran = false;
-    grid_launch(&g->control, (const void*)k_bm_grid, nblk - (g->control.absent && g->tail[w] ? 1 : 0), args, st, &ran);
+    NFX_CHECK(grid_launch(&g->control, (const void*)k_bm_grid, nblk - (g->control.absent && g->tail[w] ? 1 : 0), args,
+                          st, &ran));
     if (!ran) {  // the stepwise kernels take this and the later launches
       runs_until = w;
       break;

@@ -461,7 +461,7 @@ int el_grid_solve(MinresGrid* g, int nblk, int n, int n_blocks, const int32_t* b
   ElGridArgs a{n, n_blocks, nblk, maxit, kGridLdsBytes, brp, bci, bva, *pc, rhs, x, vec, tol, g->slots, g->res};
   void* args[] = {&a};
   bool ran = false;
-  grid_launch(&g->control, (const void*)k_el_grid, nblk - (g->control.absent ? 1 : 0), args, st, &ran);
+  NFX_CHECK(grid_launch(&g->control, (const void*)k_el_grid, nblk - (g->control.absent ? 1 : 0), args, st, &ran));
   if (!ran) return NFX_OK;
   NFX_CHECK_HIP(hipMemcpyAsync(g->h_res, g->res, sizeof(GridResult), hipMemcpyDeviceToHost, st));
   NFX_CHECK_HIP(hipStreamSynchronize(st));

@@ -26,9 +26,9 @@ constexpr int kGridThreads = 1024;
 
 // A device gives the resources of cooperative launches to one process at a time; a launch in another is
 // refused, after ~35 ms. The callers then take the stepwise kernels, and for kGridRetrySeconds they do not
-// ask again (nfx_minres_grid.hip).
+// ask that device again (nfx_backoff.h).
 constexpr int kGridRetrySeconds = 10;
-bool grid_refused();
+bool grid_refused();  // the current device
 void grid_note_refusal();
 
 // what a launch (or one system of it) reports
@@ -43,9 +43,9 @@ struct GridControl {
   int absent = 0;                      // != 0: the last block is not launched, the others give up their wait for it
   int64_t solved = 0, declined = 0;    // inner solves that ran so; that were tried so and ran stepwise
 };
-// Launches kernel on nblk blocks of kGridThreads with all their LDS. *ran = false: not launched (refused, or
-// no more allowed) and nothing ran, the stepwise kernels take it.
-void grid_launch(GridControl* c, const void* kernel, int nblk, void** args, hipStream_t st, bool* ran);
+// Launches kernel on nblk blocks of kGridThreads with all their LDS. *ran = false: not launched (refused, no
+// resources, or no more allowed) and nothing ran, the stepwise kernels take it. Any other failure is an error.
+int grid_launch(GridControl* c, const void* kernel, int nblk, void** args, hipStream_t st, bool* ran);
 constexpr int kGridMaxBlocks = 256;
 constexpr int kGridCopies = 8;
 constexpr int kGridBlockWords = 2 * kGridCopies * 2;  // 64-bit words of slots per block

@@ -9,10 +9,10 @@
 // An iteration took 10.1 us as two launches and 4.5 us here at 5,184 rows (triangles, degree 1), 14.0
 // and 7.7 at 41,088 rows (tetrahedra, degree 2), 18.7 and 8.7 at 252,288 rows (tetrahedra, degree 1).
 #include <algorithm>
-#include <atomic>
 #include <chrono>
 #include <cstdint>
 
+#include "nfx_backoff.h"
 #include "nfx_minres_grid.h"
 
 namespace nfx {
@@ -209,17 +209,19 @@ __global__ __launch_bounds__(kGridThreads) void k_minres_grid(MinresGridArgs a) 
 }
 
 namespace {
-std::atomic<int64_t> g_retry_at{0};  // steady clock, ns; any device of the process
-int64_t grid_clock() {
+GridBackoff g_backoff;
+int64_t grid_clock() {  // ns
   return std::chrono::duration_cast<std::chrono::nanoseconds>(std::chrono::steady_clock::now().time_since_epoch())
       .count();
 }
+int grid_device() {
+  int dev = -1;
+  return hipGetDevice(&dev) == hipSuccess ? dev : -1;
+}
 }  // namespace
 
-bool grid_refused() { return g_retry_at.load(std::memory_order_relaxed) > grid_clock(); }
-void grid_note_refusal() {
-  g_retry_at.store(grid_clock() + (int64_t)kGridRetrySeconds * 1000000000, std::memory_order_relaxed);
-}
+bool grid_refused() { return g_backoff.waits(grid_device(), grid_clock()); }
+void grid_note_refusal() { g_backoff.note(grid_device(), grid_clock(), (int64_t)kGridRetrySeconds * 1000000000); }
 
 int grid_clear(grid_word* slots, int nblk, GridResult* res, int n_res, hipStream_t st) {
   const int64_t words = (int64_t)nblk * kGridBlockWords;
@@ -229,16 +231,20 @@ int grid_clear(grid_word* slots, int nblk, GridResult* res, int n_res, hipStream
   return NFX_OK;
 }
 
-void grid_launch(GridControl* c, const void* kernel, int nblk, void** args, hipStream_t st, bool* ran) {
+int grid_launch(GridControl* c, const void* kernel, int nblk, void** args, hipStream_t st, bool* ran) {
   *ran = false;
-  if (c->launches == 0 || grid_refused()) return;
+  if (c->launches == 0 || grid_refused()) return NFX_OK;
   if (c->launches > 0) --c->launches;
-  if (hipLaunchCooperativeKernel(kernel, dim3(nblk), dim3(kGridThreads), args, kGridLdsBytes, st) != hipSuccess) {
-    (void)hipGetLastError();
-    grid_note_refusal();
-    return;
+  const hipError_t e = hipLaunchCooperativeKernel(kernel, dim3(nblk), dim3(kGridThreads), args, kGridLdsBytes, st);
+  const GridLaunch what = grid_outcome(e);
+  if (what != GridLaunch::ran) (void)hipGetLastError();
+  if (what == GridLaunch::error) {
+    set_error(std::string("cooperative launch: ") + hipGetErrorString(e));
+    return NFX_E_HIP;
   }
-  *ran = true;
+  if (what == GridLaunch::busy) grid_note_refusal();
+  *ran = what == GridLaunch::ran;
+  return NFX_OK;
 }
 
 // Resident blocks that the device allows (0: no cooperative launch, or too little LDS).
@@ -292,7 +298,7 @@ int minres_grid_solve(MinresGrid* g, int nblk, int lanes, int n, const int32_t* 
                   : lanes == 8 ? (const void*)k_minres_grid<8>
                                : (const void*)k_minres_grid<4>;
   bool ran = false;
-  grid_launch(&g->control, f, nblk - (g->control.absent ? 1 : 0), args, st, &ran);
+  NFX_CHECK(grid_launch(&g->control, f, nblk - (g->control.absent ? 1 : 0), args, st, &ran));
   if (!ran) return NFX_OK;
   NFX_CHECK_HIP(hipMemcpyAsync(g->h_res, g->res, sizeof(GridResult), hipMemcpyDeviceToHost, st));
   NFX_CHECK_HIP(hipStreamSynchronize(st));

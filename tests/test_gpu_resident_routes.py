@@ -398,3 +398,39 @@ def test_a_batch_is_resident_where_its_launches_pay(spec, count, resident):
     assert all(i["converged"] for i in infos)
     assert mb.resident_counts() == ((sum(i["outer"] for i in infos), 0) if resident else (0, 0))
     mb.close()
+
+
+CHILD = """
+import sys
+sys.path.insert(0, {root!r})
+from tests.test_gpu_resident_routes import _single
+s, b = _single()
+for _ in range(2):
+    x, info = s.solve(b, rtol=1e-9)
+    assert info["converged"], info
+print("counts", *s.resident_counts(), flush=True)
+s.close()
+"""
+
+
+def test_a_second_process_solves_beside_this_one():
+    """A device gives cooperative launches to one process at a time: in a second one the launch is refused and
+    the solve runs stepwise; the device is not asked again at once."""
+    import os
+    import subprocess
+    import sys
+
+    print("[routes] second process", flush=True)
+    s, b = _single()
+    s.solve(b, rtol=1e-9)
+    assert s.resident_counts()[0] > 0  # this process holds them
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    out = subprocess.run([sys.executable, "-u", "-c", CHILD.format(root=root)], capture_output=True, text=True,
+                         timeout=100)
+    print(out.stdout, out.stderr[-500:], flush=True)
+    assert out.returncode == 0, out.stderr[-2000:]
+    solved, declined = (int(v) for v in out.stdout.split("counts")[1].split())
+    assert (solved, declined) == (0, 2) or declined == 0  # refused, or the device serves both
+    x, info = s.solve(b, rtol=1e-9)
+    assert info["converged"]
+    s.close()
