@@ -720,7 +720,7 @@ int bm_grid_solve(BmGrid* g, int n_inst, int64_t n_total, const nfx_minres_batch
       (*done)[i] = 1;
       iters[i] = g->h_res[i].iters;
     }
-    ++((*done)[i] ? g->control.solved : g->control.declined);
+    grid_count(&g->control, (*done)[i] ? 0 : g->wave_of[i] < runs_until ? g->h_res[i].status : 1);
   }
   return NFX_OK;
 }

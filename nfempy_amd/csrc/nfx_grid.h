@@ -26,10 +26,9 @@ constexpr int kGridThreads = 1024;
 
 // A device gives the resources of cooperative launches to one process at a time; a launch in another is
 // refused, after ~35 ms. The callers then take the stepwise kernels, and for kGridRetrySeconds they do not
-// ask that device again (nfx_backoff.h).
+// ask that device again (nfx_backoff.h); nor after a wait that was given up, for half a second.
 constexpr int kGridRetrySeconds = 10;
 bool grid_refused();  // the current device
-void grid_note_refusal();
 
 // what a launch (or one system of it) reports
 struct GridResult {
@@ -46,6 +45,8 @@ struct GridControl {
 // Launches kernel on nblk blocks of kGridThreads with all their LDS. *ran = false: not launched (refused, no
 // resources, or no more allowed) and nothing ran, the stepwise kernels take it. Any other failure is an error.
 int grid_launch(GridControl* c, const void* kernel, int nblk, void** args, hipStream_t st, bool* ran);
+// Counts an inner solve (of an instance) by the status that its launch left, and pauses the device after 2.
+void grid_count(GridControl* c, int status);
 constexpr int kGridMaxBlocks = 256;
 constexpr int kGridCopies = 8;
 constexpr int kGridBlockWords = 2 * kGridCopies * 2;  // 64-bit words of slots per block

@@ -780,7 +780,7 @@ extern "C" int nfx_solve_minres_ir(nfx_solver* s, const int32_t* d_rowptr, const
       rc = minres_grid_solve(&s->grid, grid_blocks, s->lanes, n, d_rowptr, d_col, d_val32, d_sign, d_pc_rowptr,
                              d_pc_col, d_pc_val, rf, dx, s->buf, inner_rtol, max_inner, &it, &status, s->stream);
       if (rc) return rc;
-      ++(status ? s->grid.control.declined : s->grid.control.solved);
+      grid_count(&s->grid.control, status);
       if (status) grid_blocks = 0;
     }
     if (!grid_blocks) {
@@ -907,7 +907,7 @@ extern "C" int nfx_solve_minres_ir_tg(nfx_solver* s, const int32_t* d_rowptr, co
       rc = el_grid_solve(&s->grid, grid_blocks, n, s->b3_nblk, s->b3_rp, s->b3_ci, s->b3_va, pc, rf, dx, s->buf,
                          inner_rtol, max_inner, &it, &status, s->stream);
       if (rc) return rc;
-      ++(status ? s->grid.control.declined : s->grid.control.solved);
+      grid_count(&s->grid.control, status);
       if (status) grid_blocks = 0;
     }
     if (!grid_blocks) {
@@ -1574,6 +1574,7 @@ extern "C" int nfx_solve_minres_batch_ir(nfx_minres_batch* s, const double* d_b,
         if (done[i]) s->h_mode[i] = 2;
         rest = rest || s->h_mode[i] == 0;
       }
+      if (rest) resident = false;  // what a launch did not do once is not tried again in this solve
     }
     if (rest) {
       rc = bm_inner(s, rf, dx, tol.data(), max_inner, stepwise.data());

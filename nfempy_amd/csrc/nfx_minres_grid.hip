@@ -220,8 +220,13 @@ int grid_device() {
 }
 }  // namespace
 
+static void grid_pause() { g_backoff.note(grid_device(), grid_clock(), (int64_t)kGridRetrySeconds * 1000000000); }
 bool grid_refused() { return g_backoff.waits(grid_device(), grid_clock()); }
-void grid_note_refusal() { g_backoff.note(grid_device(), grid_clock(), (int64_t)kGridRetrySeconds * 1000000000); }
+
+void grid_count(GridControl* c, int status) {
+  ++(status ? c->declined : c->solved);
+  if (status == 2 && !c->absent) grid_pause();
+}
 
 int grid_clear(grid_word* slots, int nblk, GridResult* res, int n_res, hipStream_t st) {
   const int64_t words = (int64_t)nblk * kGridBlockWords;
@@ -242,7 +247,7 @@ int grid_launch(GridControl* c, const void* kernel, int nblk, void** args, hipSt
     set_error(std::string("cooperative launch: ") + hipGetErrorString(e));
     return NFX_E_HIP;
   }
-  if (what == GridLaunch::busy) grid_note_refusal();
+  if (what == GridLaunch::busy) grid_pause();
   *ran = what == GridLaunch::ran;
   return NFX_OK;
 }
