@@ -560,10 +560,10 @@ __global__ __launch_bounds__(kT) void k_bm_grid(BmGridArgs a) {
 
 }  // namespace
 
-int bm_grid_create(BmGrid* g, int n_inst, const nfx_minres_batch_item* items, const nfx_minres_batch_item* d_items,
-                   hipStream_t st) {
-  g->wave_of.assign(n_inst, -1);
-  g->wave_at.assign(1, 0);
+// Launches of the batch; where it can be resident, its work space. One that cannot allocates nothing.
+static int bm_grid_plan(BmGrid* g, const std::vector<int>& rows, int64_t n_total, const nfx_minres_batch_item* d_items,
+                        int32_t* scratch, hipStream_t st) {
+  const int n_inst = (int)rows.size();
   int dev = 0, coop = 0, cus = 0, per_cu = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev) != hipSuccess || !coop ||
@@ -576,9 +576,40 @@ int bm_grid_create(BmGrid* g, int n_inst, const nfx_minres_batch_item* items, co
     (void)hipGetLastError();
     return NFX_OK;
   }
-  const int cap = g->cap = std::min(cus, kGridMaxBlocks);
+  const int cap = std::min(cus, kGridMaxBlocks);
 
-  // one device and one pinned allocation
+  // entries of each instance, its blocks, and launches of at most `cap` blocks, largest instances first
+  std::vector<int32_t> nnz(n_inst);
+  hipLaunchKernelGGL(k_bm_nnz, dim3(grid_for(n_inst, 256)), dim3(256), 0, st, n_inst, d_items, scratch);
+  NFX_LAUNCH_CHECK();
+  NFX_CHECK_HIP(hipMemcpyAsync(nnz.data(), scratch, sizeof(int32_t) * n_inst, hipMemcpyDeviceToHost, st));
+  NFX_CHECK_HIP(hipStreamSynchronize(st));
+  std::vector<int> nblk(n_inst), order(n_inst);
+  for (int i = 0; i < n_inst; ++i) {
+    nblk[i] = bm_grid_blocks(rows[i], nnz[i]);
+    order[i] = i;
+    if (nblk[i] < 1 || nblk[i] > cap) return NFX_OK;
+  }
+  std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return nblk[a] > nblk[b]; });
+  std::vector<std::vector<BmGridBlock>> waves;
+  std::vector<int> wave_of(n_inst);
+  for (int i : order) {
+    size_t w = 0;
+    while (w < waves.size() && (int)waves[w].size() + nblk[i] > cap) ++w;
+    if (w == waves.size()) waves.emplace_back();
+    wave_of[i] = (int)w;
+    const int first = (int)waves[w].size();
+    for (int r = 0; r < nblk[i]; ++r) waves[w].push_back(BmGridBlock{i, r, nblk[i], first});
+  }
+  std::vector<BmGridBlock> all;
+  std::vector<int> wave_at(1, 0);
+  for (const auto& w : waves) {
+    all.insert(all.end(), w.begin(), w.end());
+    wave_at.push_back((int)all.size());
+  }
+  if (!bm_grid_pays((int)waves.size(), (int)all.size(), cap)) return NFX_OK;
+
+  // one device and one pinned allocation; without them the batch runs stepwise
   size_t at = 0;
   const auto piece = [&at](size_t bytes) {
     const size_t here = at;
@@ -587,48 +618,30 @@ int bm_grid_create(BmGrid* g, int n_inst, const nfx_minres_batch_item* items, co
   };
   const size_t o_rng = piece(sizeof(int32_t) * (size_t)n_inst * kBmRanges),
                o_slots = piece(sizeof(grid_word) * kGridSlotWords), o_res = piece(sizeof(GridResult) * n_inst),
-               o_tol = piece(sizeof(double) * n_inst),
-               o_blk = piece(sizeof(BmGridBlock) * (size_t)n_inst * kGridMaxBlocks);
-  NFX_CHECK_HIP(hipMalloc(&g->dev, at));
+               o_tol = piece(sizeof(double) * n_inst), o_blk = piece(sizeof(BmGridBlock) * all.size()),
+               o_own = piece(sizeof(float) * 3 * (size_t)n_total);
+  hipError_t e = hipMalloc(&g->dev, at);
+  at = 0;
+  const size_t h_res = piece(sizeof(GridResult) * n_inst), h_tol = piece(sizeof(double) * n_inst);
+  if (e == hipSuccess) e = hipHostMalloc(&g->host, at, hipHostMallocDefault);
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    if (g->dev) (void)hipFree(g->dev);
+    g->dev = nullptr;
+    return NFX_OK;
+  }
   g->ranges = reinterpret_cast<int32_t*>(g->dev + o_rng);
   g->slots = reinterpret_cast<grid_word*>(g->dev + o_slots);
   g->res = reinterpret_cast<GridResult*>(g->dev + o_res);
   g->tol = reinterpret_cast<double*>(g->dev + o_tol);
   g->blocks = reinterpret_cast<BmGridBlock*>(g->dev + o_blk);
-  at = 0;
-  const size_t h_res = piece(sizeof(GridResult) * n_inst), h_tol = piece(sizeof(double) * n_inst);
-  NFX_CHECK_HIP(hipHostMalloc(&g->host, at, hipHostMallocDefault));
+  g->own = reinterpret_cast<float*>(g->dev + o_own);
   g->h_res = reinterpret_cast<GridResult*>(g->host + h_res);
   g->h_tol = reinterpret_cast<double*>(g->host + h_tol);
-
-  // entries of each instance, its blocks, and launches of at most `cap` blocks, largest instances first
-  std::vector<int32_t> nnz(n_inst);
-  hipLaunchKernelGGL(k_bm_nnz, dim3(grid_for(n_inst, 256)), dim3(256), 0, st, n_inst, d_items, g->ranges);
-  NFX_LAUNCH_CHECK();
-  NFX_CHECK_HIP(hipMemcpyAsync(nnz.data(), g->ranges, sizeof(int32_t) * n_inst, hipMemcpyDeviceToHost, st));
-  NFX_CHECK_HIP(hipStreamSynchronize(st));
-  std::vector<int> nblk(n_inst), order, used;
-  for (int i = 0; i < n_inst; ++i) {
-    nblk[i] = bm_grid_blocks(items[i].n_rows, nnz[i]);
-    if (nblk[i] > 0 && nblk[i] <= cap) order.push_back(i);
-  }
-  std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return nblk[a] > nblk[b]; });
-  std::vector<std::vector<BmGridBlock>> waves;
-  for (int i : order) {
-    size_t w = 0;
-    while (w < waves.size() && (int)waves[w].size() + nblk[i] > cap) ++w;
-    if (w == waves.size()) waves.emplace_back();
-    g->wave_of[i] = (int)w;
-    const int first = (int)waves[w].size();
-    for (int r = 0; r < nblk[i]; ++r) waves[w].push_back(BmGridBlock{i, r, nblk[i], first});
-  }
-  std::vector<BmGridBlock> all;
-  for (const auto& w : waves) {
-    all.insert(all.end(), w.begin(), w.end());
-    g->wave_at.push_back((int)all.size());
-    g->tail.push_back(w.back().nblk > 1);
-  }
-  if (!all.empty()) NFX_CHECK_HIP(hipMemcpy(g->blocks, all.data(), sizeof(BmGridBlock) * all.size(), hipMemcpyHostToDevice));
+  NFX_CHECK_HIP(hipMemcpy(g->blocks, all.data(), sizeof(BmGridBlock) * all.size(), hipMemcpyHostToDevice));
+  for (const auto& w : waves) g->tail.push_back(w.back().nblk > 1);
+  g->wave_of.swap(wave_of);
+  g->wave_at.swap(wave_at);
   return NFX_OK;
 }
 
@@ -638,15 +651,18 @@ void bm_grid_destroy(BmGrid* g) {
   *g = BmGrid();
 }
 
-int bm_grid_route(BmGrid* g, int n_inst, int64_t n_total, const std::vector<nfx_batch_tg>& pc, bool* resident,
-                  hipStream_t st) {
+int bm_grid_route(BmGrid* g, const std::vector<int>& rows, int64_t n_total, const nfx_minres_batch_item* d_items,
+                  const std::vector<nfx_batch_tg>& pc, int32_t* scratch, bool* resident, hipStream_t st) {
+  const int n_inst = (int)rows.size();
   *resident = false;
   if (n_total > INT32_MAX || !g->control.launches || grid_refused()) return NFX_OK;
   // all or none: beside instances that have to iterate stepwise the others cost little there and a launch
   // each here (32 instances up to 16 x 16 x 16 cubes: 79.5 ms stepwise, 94.5 ms split)
-  for (int i = 0; i < n_inst; ++i)
-    if (g->wave_of[i] < 0) return NFX_OK;
-  if (!bm_grid_pays((int)g->wave_at.size() - 1, g->wave_at.back(), g->cap)) return NFX_OK;
+  if (!g->planned) {
+    g->planned = true;
+    NFX_CHECK(bm_grid_plan(g, rows, n_total, d_items, scratch, st));
+  }
+  if (g->wave_of.empty()) return NFX_OK;
   hipLaunchKernelGGL(k_bm_grid_zero, dim3(grid_for(n_inst * kBmRanges, 256)), dim3(256), 0, st, n_inst * kBmRanges,
                      g->ranges);
   for (size_t q = 0; q < pc.size(); ++q) {
@@ -670,7 +686,7 @@ int bm_grid_route(BmGrid* g, int n_inst, int64_t n_total, const std::vector<nfx_
 
 int bm_grid_solve(BmGrid* g, int n_inst, int64_t n_total, const nfx_minres_batch_item* d_items, const int32_t* d_mode,
                   const int32_t* h_mode, const std::vector<nfx_batch_tg>& pc, const float* rhs, float* x, float* vec,
-                  float* own, const double* tol, int maxit, int* iters, std::vector<char>* done, hipStream_t st) {
+                  const double* tol, int maxit, int* iters, std::vector<char>* done, hipStream_t st) {
   done->assign(n_inst, 0);
   const int waves = (int)g->wave_at.size() - 1;
   std::vector<char> runs(waves, 0);
@@ -690,7 +706,7 @@ int bm_grid_solve(BmGrid* g, int n_inst, int64_t n_total, const nfx_minres_batch
   a.rhs = rhs;
   a.x = x;
   a.vec = vec;
-  a.own = own;
+  a.own = g->own;
   a.tol = g->tol;
   a.slots = g->slots;
   a.res = g->res;

@@ -1242,9 +1242,10 @@ struct nfx_minres_batch {
   int32_t* act = nullptr;    // tile ids the kernels run over
   int32_t* h_act = nullptr;  // pinned staging of act
   std::vector<int32_t> h_tile_ptr;
+  std::vector<int> rows;  // of each instance
   int n_act = 0;
   int32_t* mode = nullptr;
-  float* buf = nullptr;  // 13 vectors of n_total floats
+  float* buf = nullptr;  // 10 vectors of n_total floats
   double* r64 = nullptr;
   double* pa = nullptr;  // n_tiles partials (alpha / r.r)
   double* pb = nullptr;  // n_tiles partials (y'.z / b.b)
@@ -1316,7 +1317,7 @@ extern "C" int nfx_minres_batch_create(nfx_minres_batch** out, int n_inst, const
   if (e == hipSuccess) e = hipMalloc(&s->mode, sizeof(int32_t) * n_inst);
   if (e == hipSuccess) e = hipMalloc(&s->act, sizeof(int32_t) * s->n_tiles);
   if (e == hipSuccess) e = hipHostMalloc(&s->h_act, sizeof(int32_t) * s->n_tiles, hipHostMallocDefault);
-  if (e == hipSuccess) e = hipMalloc(&s->buf, sizeof(float) * (size_t)off * 13);
+  if (e == hipSuccess) e = hipMalloc(&s->buf, sizeof(float) * (size_t)off * 10);
   if (e == hipSuccess) e = hipMalloc(&s->r64, sizeof(double) * (size_t)off);
   if (e == hipSuccess) e = hipMalloc(&s->pa, sizeof(double) * s->n_tiles);
   if (e == hipSuccess) e = hipMalloc(&s->pb, sizeof(double) * s->n_tiles);
@@ -1338,11 +1339,7 @@ extern "C" int nfx_minres_batch_create(nfx_minres_batch** out, int n_inst, const
     return NFX_E_HIP;
   }
   s->h_tile_ptr = tile_ptr;
-  const int rc = nfx::bm_grid_create(&s->grid, n_inst, items.data(), s->items, s->stream);
-  if (rc) {
-    bm_free(s);
-    return rc;
-  }
+  for (const auto& i : items) s->rows.push_back(i.n_rows);
   *out = s;
   return NFX_OK;
 }
@@ -1558,7 +1555,8 @@ extern "C" int nfx_solve_minres_batch_ir(nfx_minres_batch* s, const double* d_b,
     if (!routed) {
       rc = nfx::batch_tg_check(s->pc.data(), (int)s->pc.size());
       if (rc) return rc;
-      rc = nfx::bm_grid_route(&s->grid, m, N, s->pc, &resident, st);
+      // the sums of the residuals have been read
+      rc = nfx::bm_grid_route(&s->grid, s->rows, N, s->items, s->pc, reinterpret_cast<int32_t*>(s->sums), &resident, st);
       if (rc) return rc;
       routed = true;
     }
@@ -1567,7 +1565,7 @@ extern "C" int nfx_solve_minres_batch_ir(nfx_minres_batch* s, const double* d_b,
     bool rest = !resident;
     if (resident) {
       std::vector<char> done;
-      rc = nfx::bm_grid_solve(&s->grid, m, N, s->items, s->mode, s->h_mode, s->pc, rf, dx, s->buf, s->buf + N * 10,
+      rc = nfx::bm_grid_solve(&s->grid, m, N, s->items, s->mode, s->h_mode, s->pc, rf, dx, s->buf,
                               tol.data(), max_inner, it.data(), &done, st);
       if (rc) return rc;
       for (int i = 0; i < m; ++i) {

@@ -436,3 +436,47 @@ def test_a_second_process_solves_beside_this_one():
     x, info = s.solve(b, rtol=1e-9)
     assert info["converged"]
     s.close()
+
+
+def test_a_batch_is_planned_by_its_first_solve():
+    """Creating a batch reads none of its arrays and holds the stepwise vectors only; a system too large to be
+    resident (2 M rows) adds nothing to them when it is solved."""
+    import torch
+
+    from nfempy_amd.solvers import MinresBatch
+    from tests.test_gpu_minres_grid import _matrix
+
+    print("[routes] plan", flush=True)
+    A, d = _matrix(3000, 6, seed=1)
+    A.sort_indices()
+    dev = lambda a, t: torch.tensor(np.ascontiguousarray(a), dtype=t, device="cuda")
+    v64 = dev(A.data, torch.float64)
+    sy = {"rowptr": dev(A.indptr, torch.int32), "col": dev(A.indices, torch.int32), "vals32": v64.to(torch.float32),
+          "vals64": v64, "pinv": dev(1.0 / d, torch.float32)}
+    b = dev(np.random.default_rng(2).standard_normal(3000), torch.float64)
+    mb = MinresBatch([sy])
+    want, info = mb.solve(b)
+    mb.close()
+    rp = sy["rowptr"].clone()
+    sy["rowptr"].zero_()
+    mb = MinresBatch([sy])
+    sy["rowptr"].copy_(rp)
+    x, info2 = mb.solve(b)
+    assert mb.resident_counts() == (info2[0]["outer"], 0) and torch.equal(x, want)
+    mb.close()
+
+    print("[routes] memory", flush=True)
+    n = 2_000_000
+    ar = torch.arange(n + 1, dtype=torch.int32, device="cuda")
+    v = torch.linspace(1, 2, n, dtype=torch.float64, device="cuda")
+    sy = {"rowptr": ar, "col": ar[:-1].contiguous(), "vals32": v.to(torch.float32), "vals64": v}
+    b = torch.ones_like(v)
+    x = torch.zeros_like(b)
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    mb = MinresBatch([sy])
+    x, info = mb.solve(b, x=x)
+    used = free - torch.cuda.mem_get_info()[0]
+    assert info[0]["converged"] and mb.resident_counts() == (0, 0)
+    assert used <= 12.6 * 4 * n, used  # 10 FP32 vectors and one of FP64, and the tiles' words
+    mb.close()
