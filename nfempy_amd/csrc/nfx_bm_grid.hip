@@ -655,7 +655,7 @@ int bm_grid_route(BmGrid* g, const std::vector<int>& rows, int64_t n_total, cons
                   const std::vector<nfx_batch_tg>& pc, int32_t* scratch, bool* resident, hipStream_t st) {
   const int n_inst = (int)rows.size();
   *resident = false;
-  if (n_total > INT32_MAX || !g->control.launches || grid_refused()) return NFX_OK;
+  if (n_total > INT32_MAX || !grid_allowed(g->control)) return NFX_OK;
   // all or none: beside instances that have to iterate stepwise the others cost little there and a launch
   // each here (32 instances up to 16 x 16 x 16 cubes: 79.5 ms stepwise, 94.5 ms split)
   if (!g->planned) {

@@ -28,7 +28,6 @@ constexpr int kGridThreads = 1024;
 // refused, after ~35 ms. The callers then take the stepwise kernels, and for kGridRetrySeconds they do not
 // ask that device again (nfx_backoff.h); nor after a wait that was given up, for half a second.
 constexpr int kGridRetrySeconds = 10;
-bool grid_refused();  // the current device
 
 // what a launch (or one system of it) reports
 struct GridResult {
@@ -42,6 +41,7 @@ struct GridControl {
   int absent = 0;                      // != 0: the last block is not launched, the others give up their wait for it
   int64_t solved = 0, declined = 0;    // inner solves that ran so; that were tried so and ran stepwise
 };
+bool grid_allowed(const GridControl& c);  // a launch on the current device, now
 // Launches kernel on nblk blocks of kGridThreads with all their LDS. *ran = false: not launched (refused, no
 // resources, or no more allowed) and nothing ran, the stepwise kernels take it. Any other failure is an error.
 int grid_launch(GridControl* c, const void* kernel, int nblk, void** args, hipStream_t st, bool* ran);

@@ -564,7 +564,7 @@ extern "C" int nfx_solver_create(nfx_solver** out, int n_rows, int nnz, void* st
   hipError_t e = hipMalloc(&s->dev, at);
   at = 0;
   const size_t h_pr = piece(sizeof(double) * 2 * kResMaxBlocks), h_st = piece(sizeof(MinresState)),
-               h_res = piece(sizeof(GridResult));
+               h_res = piece(sizeof(GridResult)), h_other = piece(sizeof(int) * kGridDiagBlocks);
   if (e == hipSuccess) e = hipHostMalloc(&s->host, at, hipHostMallocDefault);
   if (e != hipSuccess) {
     set_error(std::string("nfx_solver_create: ") + hipGetErrorString(e));
@@ -582,6 +582,7 @@ extern "C" int nfx_solver_create(nfx_solver** out, int n_rows, int nnz, void* st
   s->h_partial = reinterpret_cast<double*>(s->host + h_pr);
   s->h_st = reinterpret_cast<MinresState*>(s->host + h_st);
   s->grid.h_res = reinterpret_cast<GridResult*>(s->host + h_res);
+  s->grid.h_other = reinterpret_cast<int*>(s->host + h_other);
   *out = s;
   return NFX_OK;
 }
@@ -761,13 +762,16 @@ extern "C" int nfx_solve_minres_ir(nfx_solver* s, const int32_t* d_rowptr, const
   int total = 0, outer = 0;
   double rel = 0;
   const int g = grid_for(n, kBlock);
-  // inner solves as one resident launch where the system fits the CUs' LDS, stepwise else and after
-  // a launch that could not do it (preconditioner not diagonal, blocks not resident in time)
-  int grid_blocks = s->b3_va ? 0 : minres_grid_blocks(&s->grid, n, s->nnz);
+  // inner solves as one resident launch where the system fits the CUs' LDS and the preconditioner is
+  // diagonal, stepwise else and after a launch that did not do it
+  int grid_blocks = s->b3_va || !grid_allowed(s->grid.control) ? 0 : minres_grid_blocks(&s->grid, n, s->nnz);
+  const bool ask = grid_blocks != 0;
+  if (ask) NFX_CHECK(minres_grid_ask(&s->grid, n, d_pc_rowptr, d_pc_col, s->stream));
   for (; outer <= max_outer; ++outer) {
     double rr = 0, bb = 0;
     int rc = residual64(s, d_rowptr, d_col, d_val64, d_x, d_b, &rr, &bb);
     if (rc) return rc;
+    if (outer == 0 && ask && !minres_grid_diagonal(&s->grid)) grid_blocks = 0;
     const double rn = sqrt(rr), bn = sqrt(bb);
     rel = bn > 0 ? rn / bn : rn;
     if (h_hist && outer < hist_cap) h_hist[outer] = rel;
@@ -888,7 +892,7 @@ extern "C" int nfx_solve_minres_ir_tg(nfx_solver* s, const int32_t* d_rowptr, co
   double rel = 0;
   const int g = grid_for(n, kBlock);
   // as one resident launch where the block operator and the preconditioner fit the CUs' LDS
-  int grid_blocks = s->b3_va ? el_grid_blocks(el_grid_capacity(), pc, s->b3_nblk) : 0;
+  int grid_blocks = s->b3_va && grid_allowed(s->grid.control) ? el_grid_blocks(el_grid_capacity(), pc, s->b3_nblk) : 0;
   for (; outer <= max_outer; ++outer) {
     double rr = 0, bb = 0;
     int rc = residual64(s, d_rowptr, d_col, d_val64, d_x, d_b, &rr, &bb);

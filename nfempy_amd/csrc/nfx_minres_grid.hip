@@ -76,7 +76,7 @@ __global__ __launch_bounds__(kGridThreads) void k_minres_grid(MinresGridArgs a) 
   const int64_t base = 4 * (int64_t)nz + 4 * (int64_t)(R + 1) + 4 * (int64_t)((nz + 1) / 2);
   const int nw = (n + 31) >> 5;
   bool fits = base + 8 * (int64_t)nw <= a.lds;
-  bool diag = true;
+  bool diag = true;  // known to the host (k_grid_diagonal); pva is indexed by it
   for (int i = t; i < R; i += T) {
     const int j = a.prp[r0 + i];
     diag = diag && a.prp[r0 + i + 1] == j + 1 && a.pci[j] == r0 + i;
@@ -221,7 +221,7 @@ int grid_device() {
 }  // namespace
 
 static void grid_pause() { g_backoff.note(grid_device(), grid_clock(), (int64_t)kGridRetrySeconds * 1000000000); }
-bool grid_refused() { return g_backoff.waits(grid_device(), grid_clock()); }
+bool grid_allowed(const GridControl& c) { return c.launches != 0 && !g_backoff.waits(grid_device(), grid_clock()); }
 
 void grid_count(GridControl* c, int status) {
   ++(status ? c->declined : c->solved);
@@ -238,7 +238,7 @@ int grid_clear(grid_word* slots, int nblk, GridResult* res, int n_res, hipStream
 
 int grid_launch(GridControl* c, const void* kernel, int nblk, void** args, hipStream_t st, bool* ran) {
   *ran = false;
-  if (c->launches == 0 || grid_refused()) return NFX_OK;
+  if (!grid_allowed(*c)) return NFX_OK;
   if (c->launches > 0) --c->launches;
   const hipError_t e = hipLaunchCooperativeKernel(kernel, dim3(nblk), dim3(kGridThreads), args, kGridLdsBytes, st);
   const GridLaunch what = grid_outcome(e);
@@ -289,6 +289,28 @@ int minres_grid_blocks(const MinresGrid* g, int n, int64_t nnz) {
     if (bytes / nblk <= spare && (6 * nnz + 4 * (int64_t)n) / nblk + n / 4 <= spare) return nblk;
   }
   return 0;
+}
+
+// one flag a block, written to the host: the answer comes with whatever the stream is waited for next
+__global__ __launch_bounds__(256) void k_grid_diagonal(int n, const int32_t* __restrict__ prp,
+                                                       const int32_t* __restrict__ pci, int* __restrict__ other) {
+  bool diag = true;
+  for (int64_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += kGridDiagBlocks * 256) {
+    const int j = prp[i];
+    diag = diag && prp[i + 1] == j + 1 && pci[j] == i;
+  }
+  const int all = __syncthreads_and(diag);
+  if (threadIdx.x == 0) other[blockIdx.x] = !all;
+}
+
+int minres_grid_ask(MinresGrid* g, int n, const int32_t* prp, const int32_t* pci, hipStream_t st) {
+  hipLaunchKernelGGL(k_grid_diagonal, dim3(kGridDiagBlocks), dim3(256), 0, st, n, prp, pci, g->h_other);
+  NFX_LAUNCH_CHECK();
+  return NFX_OK;
+}
+
+bool minres_grid_diagonal(const MinresGrid* g) {
+  return std::none_of(g->h_other, g->h_other + kGridDiagBlocks, [](int o) { return o != 0; });
 }
 
 int minres_grid_solve(MinresGrid* g, int nblk, int lanes, int n, const int32_t* rp, const int32_t* ci, const float* va,

@@ -262,13 +262,13 @@ def test_stepwise_where_no_launch_is_allowed():
     assert outer > 1 and s.resident_counts() == (outer, 0)
     s.set_resident(0)
     x, info = s.solve(b, rtol=1e-10)
-    assert info["converged"] and s.resident_counts() == (outer, 1)
+    assert info["converged"] and s.resident_counts() == (outer, 0)
     s.set_resident(1)  # the second inner solve is declined
     x, info = s.solve(b, rtol=1e-10)
-    assert info["converged"] and s.resident_counts() == (outer + 1, 2)
+    assert info["converged"] and s.resident_counts() == (outer + 1, 1)
     s.set_resident()
     x, info = s.solve(b, rtol=1e-10)
-    assert s.resident_counts() == (2 * outer + 1, 2) and bool((x == full).all())
+    assert s.resident_counts() == (2 * outer + 1, 1) and bool((x == full).all())
     s.close()
 
     print("[routes] elasticity", flush=True)
@@ -432,7 +432,7 @@ def test_a_second_process_solves_beside_this_one():
     print(out.stdout, out.stderr[-500:], flush=True)
     assert out.returncode == 0, out.stderr[-2000:]
     solved, declined = (int(v) for v in out.stdout.split("counts")[1].split())
-    assert (solved, declined) == (0, 2) or declined == 0  # refused, or the device serves both
+    assert (solved, declined) == (0, 1) or declined == 0  # refused once, or the device serves both
     x, info = s.solve(b, rtol=1e-9)
     assert info["converged"]
     s.close()
