@@ -443,10 +443,12 @@ struct RowLoad {
   uint32_t pw[2];  // packed column positions (row_pos_packed)
 };
 
-// RS_ONLY: st holds only Rs | Bc | ck (the per-element path; tiles with per-quadrature
-// coefficients are not processed). n_in_tile: rows of this tile (at most TILE * RPT).
+// PART: the part of the reference table that st holds. kTabRef: Rs | Bc | ck, one coefficient per element (tiles
+// with per-quadrature coefficients are not processed); kTabQuad: the values at the quadrature points, for those.
+// n_in_tile: rows of this tile (at most TILE * RPT).
+constexpr int kTabAll = 0, kTabRef = 1, kTabQuad = 2;
 template <int DIM, int NB, int NP, int NQ, int TILE, typename R, bool GEO = false, int RPT = 1,
-          bool RS_ONLY = false, bool OFF_PACKED = false>
+          int PART = kTabAll, bool OFF_PACKED = false>
 __device__ __forceinline__ void darcy_row_tile(
     int r0, int n_rows, const int32_t* __restrict__ inc, const uint8_t* __restrict__ pos,
     const int32_t* __restrict__ rowptr, const uint32_t* __restrict__ signs,
@@ -459,19 +461,19 @@ __device__ __forceinline__ void darcy_row_tile(
   constexpr int NT = DarcyTab<DIM, NB, NP, NQ>::NT;
   constexpr int NT_RS = NQ * (1 + NB * DIM + NB + NP);  // start of Rs | Bc | ck
   const int rl = min(r0 + n_in_tile, n_rows);
-  const bool per_element = (ks_q == 0 && fs_q == 0);
-  if (RS_ONLY && !per_element) return;
+  const bool per_element = PART != kTabQuad && ks_q == 0 && fs_q == 0;
+  if (PART == kTabRef && !per_element) return;
   const R* tw = st;
   const R* tphi = st + NQ;
   const R* tdiv = tphi + NQ * NB * DIM;
   const R* tpsi = tdiv + NQ * NB;
-  const R* tRs = RS_ONLY ? st : tpsi + NQ * NP;
+  const R* tRs = PART == kTabRef ? st : tpsi + NQ * NP;
   const R* tBc = tRs + NB * NB * NS;
   const R* tck = tBc + NB * NP;
   RowLoad<DIM, R, GEO> in[RPT];
-  // column positions of the longer rows, five words an incidence: with the incidences, ahead of the
-  // loads that depend on those (RS_ONLY: registers are left for them)
-  constexpr bool POS_EARLY = RS_ONLY && RPT == 1 && !row_pos_packed(NL) && row_pos_stride(NL) % 4 == 0;
+  // column positions of the longer rows, NPW words an incidence: with the incidences, ahead of the
+  // loads that depend on those (kTabRef: registers are left for them)
+  constexpr bool POS_EARLY = PART == kTabRef && RPT == 1 && !row_pos_packed(NL) && row_pos_stride(NL) % 4 == 0;
   constexpr int NPW = POS_EARLY ? row_pos_stride(NL) / 4 : 1;
   uint32_t pwd[2][NPW];
   int off_early = 0;
@@ -549,8 +551,10 @@ __device__ __forceinline__ void darcy_row_tile(
   // the reference-tensor path reads only Rs | Bc | ck; a caller that already holds the
   // table in st (same element, same path) passes load_table = false
   if (load_table) {
-    if constexpr (RS_ONLY) {
+    if constexpr (PART == kTabRef) {
       for (int i = threadIdx.x; i < NT - NT_RS; i += TILE) st[i] = tab[NT_RS + i];
+    } else if constexpr (PART == kTabQuad) {
+      for (int i = threadIdx.x; i < NT_RS; i += TILE) st[i] = tab[i];
     } else {
       for (int i = (per_element ? NT_RS : 0) + threadIdx.x; i < NT; i += TILE) st[i] = tab[i];
     }
@@ -587,7 +591,7 @@ __device__ __forceinline__ void darcy_row_tile(
       R row[NL];
 #pragma unroll
       for (int b = 0; b < NL; ++b) row[b] = 0;
-      if (RS_ONLY || per_element) {
+      if (PART == kTabRef || per_element) {
         if (aj < NB) {
           R gs[NS];
 #pragma unroll
@@ -608,7 +612,7 @@ __device__ __forceinline__ void darcy_row_tile(
           for (int b = 0; b < NB; ++b) row[b] = tBc[b * NP + k];
           res -= L.dj[j] * L.fv[j] * tck[k];
         }
-      } else if (!RS_ONLY && aj < NB) {
+      } else if (PART != kTabRef && aj < NB) {
         // symmetric G / detJ from the packed upper triangle
         R Gd[DIM][DIM];
         {
@@ -644,7 +648,7 @@ __device__ __forceinline__ void darcy_row_tile(
 #pragma unroll
           for (int k = 0; k < NP; ++k) row[NB + k] -= wd * tpsi[q * NP + k];
         }
-      } else if (!RS_ONLY) {
+      } else if (PART != kTabRef) {
         const int k = aj - NB;
         for (int q = 0; q < NQ; ++q) {
           const R wp = tw[q] * tpsi[q * NP + k];
@@ -719,7 +723,7 @@ constexpr int row_kernel_min_waves() {
   return (NB <= 4 && sizeof(R) == 4) ? 8 : 1;
 }
 
-template <int DIM, int NB, int NP, int NQ, typename R, bool GEO, bool RS_ONLY = false>
+template <int DIM, int NB, int NP, int NQ, typename R, bool GEO, int PART = kTabAll>
 __global__ __launch_bounds__(kRowsPerBlock)
 __attribute__((amdgpu_waves_per_eu(row_kernel_min_waves<NB, R>(), 8))) void k_darcy_rows(
     int n_rows, const int32_t* __restrict__ inc, const uint8_t* __restrict__ pos,
@@ -729,7 +733,8 @@ __attribute__((amdgpu_waves_per_eu(row_kernel_min_waves<NB, R>(), 8))) void k_da
     R* __restrict__ vals, R* __restrict__ rhs, DarcyRowBc<R> bc, const R* __restrict__ geo,
     const int32_t* __restrict__ tile_map, int n_map) {
   constexpr int NL = NB + NP;
-  constexpr int NT = DarcyTab<DIM, NB, NP, NQ>::NT - (RS_ONLY ? NQ * (1 + NB * DIM + NB + NP) : 0);
+  constexpr int NQV = NQ * (1 + NB * DIM + NB + NP);  // values at the quadrature points
+  constexpr int NT = PART == kTabQuad ? NQV : DarcyTab<DIM, NB, NP, NQ>::NT - (PART == kTabRef ? NQV : 0);
   constexpr int RPT = row_kernel_rpt<NB, R>();
   __shared__ R st[NT];
   __shared__ R sv[kRowsPerBlock * RPT * 2 * NL];
@@ -743,7 +748,7 @@ __attribute__((amdgpu_waves_per_eu(row_kernel_min_waves<NB, R>(), 8))) void k_da
   if constexpr (NB <= 4) {
     const int t = tile_map ? tile_map[blockIdx.x] : (int)blockIdx.x;
     if (t < 0 || t >= n_tiles) return;
-    darcy_row_tile<DIM, NB, NP, NQ, kRowsPerBlock, R, GEO, RPT, false, row_off_packed(NB + NP) && RPT == 1>(
+    darcy_row_tile<DIM, NB, NP, NQ, kRowsPerBlock, R, GEO, RPT, kTabAll, row_off_packed(NB + NP) && RPT == 1>(
         t * kRowsPerBlock * RPT, n_rows, inc, pos, rowptr, signs, cells, coords, tab, kinv, ks_e, ks_q, f, fs_e,
         fs_q, vals, rhs, st, sv, bc, true, geo);
   } else {
@@ -752,7 +757,7 @@ __attribute__((amdgpu_waves_per_eu(row_kernel_min_waves<NB, R>(), 8))) void k_da
     for (int i = blockIdx.x; i < n_slots; i += gridDim.x) {
       const int t = tile_map ? tile_map[i] : i;
       if (t < 0 || t >= n_tiles) continue;
-      darcy_row_tile<DIM, NB, NP, NQ, kRowsPerBlock, R, GEO, RPT, RS_ONLY>(t * kRowsPerBlock * RPT, n_rows, inc, pos,
+      darcy_row_tile<DIM, NB, NP, NQ, kRowsPerBlock, R, GEO, RPT, PART>(t * kRowsPerBlock * RPT, n_rows, inc, pos,
                                                                   rowptr, signs, cells, coords, tab, kinv, ks_e,
                                                                   ks_q, f, fs_e, fs_q, vals, rhs, st, sv, bc,
                                                                   first, geo);
@@ -858,7 +863,7 @@ __attribute__((amdgpu_waves_per_eu(batched_min_waves<KD>(), 8))) void k_darcy_ro
         held_tab = nullptr;  // nothing loaded: the next tile reloads the table
         continue;
       }
-      darcy_row_tile<3, 15, 4, 27, TILE, float, true, 1, true>(
+      darcy_row_tile<3, 15, 4, 27, TILE, float, true, 1, kTabRef>(
             tl.y, it.n_rows, inc, pos, rowptr, signs, cells, coords, tab, kinv, it.ks_e, it.ks_q, f, it.fs_e,
             it.fs_q, vals, rhs, st, sv, no_bc, load, geo, tile_n);
     }
@@ -905,10 +910,10 @@ static int launch_darcy_rows(int n_rows, const int32_t* inc, const uint8_t* pos,
     // 32.3, and 116 registers instead of 166; 6 blocks a CU instead of 5: 42.5 us instead of 45.8), and as
     // many blocks as are resident at once: on 41,154 tetrahedra, 4,227 tiles, 36.0 us with these 1,536
     // blocks, 39.3 with 1,280, 41.3 with 2,048 (a third of them start when the others end), 37.4 with one
-    // tile a block. The sums over quadrature points are uneven from tile to tile: 105 us with 2,048
-    // blocks, 122 so.
+    // tile a block. The sums over quadrature points (below; only the values there in LDS: 106.5 us -> 96.9,
+    // in FP64 on 14 cubed 147 -> 77) are uneven from tile to tile: 105 us with 2,048 blocks, 122 so.
     if (geo && ksq == 0 && fsq == 0) {
-      constexpr auto kernel = k_darcy_rows<DIM, NB, NP, NQ, R, true, true>;
+      constexpr auto kernel = k_darcy_rows<DIM, NB, NP, NQ, R, true, kTabRef>;
       static const int resident = resident_blocks((const void*)kernel);
       launch(kernel, resident, metric);
       NFX_LAUNCH_CHECK();
@@ -916,7 +921,7 @@ static int launch_darcy_rows(int n_rows, const int32_t* inc, const uint8_t* pos,
     }
   }
   if (geo)
-    launch(k_darcy_rows<DIM, NB, NP, NQ, R, true>, 2048, metric);
+    launch(k_darcy_rows<DIM, NB, NP, NQ, R, true, (NB > 4 ? kTabQuad : kTabAll)>, 2048, metric);
   else
     launch(k_darcy_rows<DIM, NB, NP, NQ, R, false>, 2048, nullptr);
   NFX_LAUNCH_CHECK();
