@@ -13,6 +13,8 @@
 //   rhsrow  int32 (NP, E)           pressure residual rows
 //   tables  R: w[NQ] | phi[NQ][NB][DIM] | div[NQ][NB] | psi[NQ][NP]
 // One thread assembles one element; the element matrix never leaves registers.
+#include <atomic>
+
 #include "nfx_common.h"
 
 namespace nfx {
@@ -870,17 +872,26 @@ __attribute__((amdgpu_waves_per_eu(batched_min_waves<KD>(), 8))) void k_darcy_ro
   }
 }
 
-// Blocks of a row kernel that the device holds at once (every GPU the library runs on is alike).
-static int resident_blocks(const void* kernel) {
+// Blocks of a row kernel that the current device holds at once; `held` keeps them for a kernel, per device.
+constexpr int kHeldDevices = 64;
+static int resident_blocks(const void* kernel, std::atomic<int> (&held)[kHeldDevices]) {
   int dev = 0, cus = 0, per_cu = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+  if (hipGetDevice(&dev) != hipSuccess) {
+    (void)hipGetLastError();
+    return 2048;
+  }
+  const bool in_table = dev >= 0 && dev < kHeldDevices;
+  int n = in_table ? held[dev].load(std::memory_order_relaxed) : 0;
+  if (n) return n;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
       hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kRowsPerBlock, 0) != hipSuccess || cus < 1 ||
       per_cu < 1) {
     (void)hipGetLastError();
     return 2048;
   }
-  return cus * per_cu;
+  n = cus * per_cu;
+  if (in_table) held[dev].store(n, std::memory_order_relaxed);
+  return n;
 }
 
 template <int DIM, int NB, int NP, int NQ, typename R>
@@ -914,8 +925,8 @@ static int launch_darcy_rows(int n_rows, const int32_t* inc, const uint8_t* pos,
     // in FP64 on 14 cubed 147 -> 77) are uneven from tile to tile: 105 us with 2,048 blocks, 122 so.
     if (geo && ksq == 0 && fsq == 0) {
       constexpr auto kernel = k_darcy_rows<DIM, NB, NP, NQ, R, true, kTabRef>;
-      static const int resident = resident_blocks((const void*)kernel);
-      launch(kernel, resident, metric);
+      static std::atomic<int> held[kHeldDevices];
+      launch(kernel, resident_blocks((const void*)kernel, held), metric);
       NFX_LAUNCH_CHECK();
       return NFX_OK;
     }
