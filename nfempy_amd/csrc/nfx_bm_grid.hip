@@ -21,7 +21,6 @@ namespace nfx {
 namespace {
 
 constexpr int kT = kGridThreads;
-constexpr int kBmGridCheck = 16;   // iterations between stopping tests, as in the stepwise solver
 constexpr int kBmGridAgg = 128;    // coarse unknowns of an instance: 16 inverse entries a thread
 // Bytes of an instance (6 an entry, 40 a row) per block: what leaves room for the values in LDS. Half of
 // it is no faster (the sums over twice the blocks take longer) and fills two launches instead of one.
@@ -91,9 +90,6 @@ template <int J>
 __device__ __forceinline__ float quad(float v) {
   return dpp_move<J * 0x55>(v);
 }
-
-// a value that all threads share, in a scalar register
-__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
 // row of a cell block (w) times the cell's values, one per lane of its NB lanes
 template <int NB>
@@ -356,21 +352,20 @@ __device__ __forceinline__ void bm_grid_run(const BmGridArgs& a, const BmGridBlo
         acc += (double)(s * zc[i]) * (double)y;
       }
       grid_post(g, acc);
-      // the rotation, and every kBmGridCheck iterations the test of the estimate after k - 1 of them
+      // the rotation, and every kGridCheck iterations the test of the estimate after k - 1 of them
       MinresState st;
       minres_scalars(sts[(k + 1) & 1], st, beta, k == 1);
       if (t == 0) sts[k & 1] = st;  // read after the next barrier only
       const bool last = !(beta > 0) || k - 1 >= a.maxit ||
-                        (k > 1 && (k - 1) % kBmGridCheck == 0 && st.phibar <= a.tol[bl.inst] * st.beta1);
+                        (k > 1 && (k - 1) % kGridCheck == 0 && st.phibar <= a.tol[bl.inst] * st.beta1);
       if (k > 1) {
-        const float sprev = st.oldb > 0 ? (float)(1.0 / st.oldb) : 0.f;
-        const float oldeps = (float)st.oldeps, delta = (float)st.delta, denom = (float)st.denom, phi = (float)st.phi;
+        const MinresStep step(st);
         for (int i = t; i < R; i += kT) {
           const int r = rid[i];
-          const float w1 = wb[r], w = (zp[r] * sprev - oldeps * wa[r] - delta * w1) * denom;
+          const float w1 = wb[r], w = step.w(zp[r], wa[r], w1);
           wa[r] = w1;
           wb[r] = w;
-          xv[r] += phi * w;
+          xv[r] += step.phi * w;
           zp[r] = zc[i];
         }
       } else {

@@ -20,7 +20,6 @@ namespace nfx {
 namespace {
 
 constexpr int kT = kGridThreads;
-constexpr int kElGridCheck = 16;   // iterations between stopping tests, as in the stepwise solver
 constexpr int kElGridAgg = 128;    // aggregates (the coarse vector and its pieces are in LDS)
 constexpr int kElGridCells = kT / 30;  // cells of a block: 5 blocks x 6 components, a thread each
 
@@ -35,8 +34,6 @@ struct ElGridArgs {
   grid_word* slots;
   GridResult* res;
 };
-
-__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
 __global__ __launch_bounds__(kT) void k_el_grid(ElGridArgs a) {
   extern __shared__ __align__(16) char lds[];
@@ -275,21 +272,20 @@ __global__ __launch_bounds__(kT) void k_el_grid(ElGridArgs a) {
         acc += (double)(s * zc[x]) * (double)y;
       }
       grid_post(g, acc);
-      // the rotation, and every kElGridCheck iterations the test of the estimate after k - 1 of them
+      // the rotation, and every kGridCheck iterations the test of the estimate after k - 1 of them
       MinresState st;
       minres_scalars(sts[(k + 1) & 1], st, beta, k == 1);
       if (t == 0) sts[k & 1] = st;  // read after the next barrier only
       const bool last = !(beta > 0) || k - 1 >= a.maxit ||
-                        (k > 1 && (k - 1) % kElGridCheck == 0 && st.phibar <= a.tol * st.beta1);
-      const float sprev = st.oldb > 0 ? (float)(1.0 / st.oldb) : 0.f;
-      const float oldeps = (float)st.oldeps, delta = (float)st.delta, denom = (float)st.denom, phi = (float)st.phi;
+                        (k > 1 && (k - 1) % kGridCheck == 0 && st.phibar <= a.tol * st.beta1);
+      const MinresStep step(st);
       for (int x = t; x < R; x += kT) {
         if (k > 1) {
           const int r = grow(x);
-          const float w1 = wb[r], w = (zp[x] * sprev - oldeps * wa[r] - delta * w1) * denom;
+          const float w1 = wb[r], w = step.w(zp[x], wa[r], w1);
           wa[r] = w1;
           wb[r] = w;
-          a.x[r] += phi * w;
+          a.x[r] += step.phi * w;
         }
         zp[x] = zc[x];
       }

@@ -47,6 +47,7 @@ bool grid_allowed(const GridControl& c);  // a launch on the current device, now
 int grid_launch(GridControl* c, const void* kernel, int nblk, void** args, hipStream_t st, bool* ran);
 // Counts an inner solve (of an instance) by the status that its launch left, and pauses the device after 2.
 void grid_count(GridControl* c, int status);
+constexpr int kGridCheck = 16;  // iterations between tests of the estimate, as in the stepwise solvers
 constexpr int kGridMaxBlocks = 256;
 constexpr int kGridCopies = 8;
 constexpr int kGridBlockWords = 2 * kGridCopies * 2;  // 64-bit words of slots per block
@@ -179,6 +180,9 @@ __device__ __forceinline__ bool grid_wait(GridSync& g, double& sum) {
   }
   return ok;
 }
+
+// a value that all threads share, in a scalar register
+__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
 // The columns that a block's rows meet, as a list, and the rows' columns as 16-bit places in it.
 // Row i has entries start(i) .. start(i) + rowp[i + 1] - rowp[i] of ci; n columns in all.

@@ -65,4 +65,19 @@ __device__ __forceinline__ void minres_scalars(const MinresState& in, MinresStat
   if (!(beta > 0)) out.stop = 1;
 }
 
+// The update of iteration k - 1 from the scalars that minres_scalars left for it, in FP32: w from z of that
+// iteration and the two w before it, x += phi w.
+struct MinresStep {
+  float sprev, oldeps, delta, denom, phi;
+  __device__ __forceinline__ explicit MinresStep(const MinresState& st)
+      : sprev(st.oldb > 0 ? (float)(1.0 / st.oldb) : 0.f),
+        oldeps((float)st.oldeps),
+        delta((float)st.delta),
+        denom((float)st.denom),
+        phi((float)st.phi) {}
+  __device__ __forceinline__ float w(float z, float wa, float wb) const {
+    return (z * sprev - oldeps * wa - delta * wb) * denom;
+  }
+};
+
 }  // namespace nfx

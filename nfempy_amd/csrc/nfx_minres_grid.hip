@@ -17,8 +17,6 @@
 
 namespace nfx {
 
-constexpr int kGridCheck = 16;  // iterations between tests of the estimate, as in the stepwise solver
-
 struct MinresGridArgs {
   int n, nblk, maxit, lds;
   const int32_t *rp, *ci;
@@ -172,13 +170,12 @@ __global__ __launch_bounds__(kGridThreads) void k_minres_grid(MinresGridArgs a) 
     const MinresState in = st;
     minres_scalars(in, st, beta, k == 1);
     if (k > 1) {
-      const float sprev = st.oldb > 0 ? (float)(1.0 / st.oldb) : 0.f;
-      const float oldeps = (float)st.oldeps, delta = (float)st.delta, denom = (float)st.denom, phi = (float)st.phi;
+      const MinresStep step(st);
       for (int i = t; i < R; i += T) {
-        const float w = (zp[i] * sprev - oldeps * wa[i] - delta * wb[i]) * denom;
+        const float w = step.w(zp[i], wa[i], wb[i]);
         wa[i] = wb[i];
         wb[i] = w;
-        xv[i] += phi * w;
+        xv[i] += step.phi * w;
       }
     }
     if (last) break;
