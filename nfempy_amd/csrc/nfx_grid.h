@@ -10,6 +10,14 @@
 //  * a vector: stored and loaded with relaxed device-scope accesses (they pass the caches that are not
 //    coherent between XCDs); a block waits for its stores before it posts the next sum.
 // Device-scope fences instead of these accesses cost 5-30 us per step (measured, 8-256 blocks).
+//
+// That is no release / acquire pair of the language: the accesses are relaxed, and a thread's vector stores come
+// before its block's post only by what this GPU does with them. Relied on, in what hipcc makes of them for gfx950
+// (global_store / global_load with sc1, no cache write-back or invalidate): a device-scope store is written
+// through the XCD's L2, and counts in vmcnt until it is where every XCD's device-scope load finds it; such a load
+// does not return an older line of its own L2; and a load is not issued before the barrier that ends the wait
+// for the post. A wait for vmcnt(0) in every wave and a barrier stand between the stores and the post. Vectors
+// that other blocks read go through grid_store and grid_load only; plain accesses are to a block's own rows.
 // Two slot sets alternate: a block posts step k + 2 only after every block has read step k.
 //
 // Every wait is bounded (kGridWaitTicks): a block that gives up leaves, the others then give up in
