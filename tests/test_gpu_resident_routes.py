@@ -480,3 +480,28 @@ def test_a_batch_is_planned_by_its_first_solve():
     assert info[0]["converged"] and mb.resident_counts() == (0, 0)
     assert used <= 12.6 * 4 * n, used  # 10 FP32 vectors and one of FP64, and the tiles' words
     mb.close()
+
+
+@pytest.mark.parametrize("n", [1, 2, 4])
+def test_elasticity_solution_against_a_direct_solve(n):
+    """The resident solve against scipy's sparse LU of the same FP64 matrix: an error is at most the residual
+    over the smallest eigenvalue in magnitude (the matrix is symmetric)."""
+    import scipy.sparse as sps
+    import scipy.sparse.linalg as spla
+
+    print(f"[routes] elasticity against LU n={n}", flush=True)
+    y = _elasticity(n)
+    x, info = y.solve(rtol=1e-10)
+    assert info["converged"] and y.last_resident == (info["outer"], 0)
+    rp, col, _, v64 = (v.cpu().numpy() for v in y.full("A"))
+    A = sps.csc_matrix(sps.csr_matrix((v64, col, rp), shape=(y.n, y.n)))
+    assert abs(A - A.T).max() <= 1e-13 * abs(A).max()
+    b = -y.rhs64.cpu().numpy()
+    lu = spla.splu(A)
+    want = lu.solve(b)
+    want += lu.solve(b - A @ want)
+    inverse = spla.LinearOperator(A.shape, matvec=lu.solve, dtype=np.float64)
+    lowest = abs(spla.eigsh(A, k=1, sigma=0.0, OPinv=inverse, which="LM", return_eigenvectors=False)[0])
+    err, bound = np.linalg.norm(x.cpu().numpy() - want), 1e-10 * np.linalg.norm(b) / lowest
+    print(f"[routes] error {err:.2e}, bound {bound:.2e}, |x| {np.linalg.norm(want):.2e}", flush=True)
+    assert err <= 1.1 * bound
