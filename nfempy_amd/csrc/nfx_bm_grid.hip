@@ -10,7 +10,7 @@
 // where the stepwise kernels need eight launches over the whole batch. Without a cycle (diagonal
 // preconditioner) the middle one falls away; the learned smoother's couplings add two, for x1 and t2.
 // Bound by the exchanges (1.2-2.6 us each, and ~1 us for what is then loaded) and the product. Twelve
-// instances of 384-4,374 cells, both degrees: 70 us an iteration stepwise, 19 us here; the largest (58,320
+// instances of 384-4,374 cells, both degrees: 70 us an iteration stepwise, 17.5 us here; the largest (58,320
 // rows, 1.5 M entries, 87 blocks) alone takes 18 us with the cycle and 10 us without.
 #include <algorithm>
 #include <climits>

@@ -8,7 +8,7 @@
 //   z | y = A z, alpha | y', x1 = W y' of the cells and, again, of their neighbours, t1 = y' - S x1 and
 //   its sums over the aggregates (a piece per block) | the coarse values that the block needs,
 //   z = x1 + P y + W (t1 - S P y), y'.z
-// where the stepwise solver has five launches: 31.9 and 16.7 us an iteration at 3,072 cells (77,184 rows),
+// where the stepwise solver has five launches: 31.9 and 15.6-16.7 us an iteration at 3,072 cells (77,184 rows),
 // of which the exchanges with the loads after them take ~12.
 #include <algorithm>
 #include <climits>
