@@ -353,7 +353,8 @@ int nfx_solver_create(nfx_solver** out, int n_rows, int nnz, void* stream);
 int nfx_solver_destroy(nfx_solver* s);
 /* Resident solves. An inner solve of a system that fits the compute units' local memory runs as one
  * cooperative launch where the device gives one, stepwise (a few launches an iteration) otherwise; the two
- * differ by roundings. launches: how many resident launches the object may still make (-1: any number, the
+ * differ by roundings. A device gives them to one process at a time: after a refusal, or a launch whose blocks
+ * gave up waiting for each other, solves on that device run stepwise for ten seconds. launches: how many resident launches the object may still make (-1: any number, the
  * default; 0: stepwise only). absent != 0 (for tests of what follows): launches leave out their last block,
  * so that the others of its system give up waiting for it after half a second, as they do where the device
  * does not run them all, and the solve goes on stepwise. h_counts (2 values), since creation: inner solves
