@@ -354,11 +354,12 @@ int nfx_solver_destroy(nfx_solver* s);
 /* Resident solves. An inner solve of a system that fits the compute units' local memory runs as one
  * cooperative launch where the device gives one, stepwise (a few launches an iteration) otherwise; the two
  * differ by roundings. A device gives them to one process at a time: after a refusal, or a launch whose blocks
- * gave up waiting for each other, solves on that device run stepwise for ten seconds. launches: how many resident launches the object may still make (-1: any number, the
- * default; 0: stepwise only). absent != 0 (for tests of what follows): launches leave out their last block,
- * so that the others of its system give up waiting for it after half a second, as they do where the device
- * does not run them all, and the solve goes on stepwise. h_counts (2 values), since creation: inner solves
- * that ran resident, and those that were tried so and ran stepwise. */
+ * gave up waiting for each other, solves on that device run stepwise for ten seconds. launches: how many
+ * resident launches the object may still make (-1: any number, the default; 0: stepwise only). absent != 0 (for
+ * tests of what follows): launches leave out their last block, so that the others of its system give up waiting
+ * for it after half a second, as they do where the device does not run them all, and the solve goes on
+ * stepwise. h_counts (2 values), since creation: inner solves that ran resident, and those that were tried so
+ * and ran stepwise. */
 int nfx_solver_set_resident(nfx_solver* s, int64_t launches, int absent);
 int nfx_solver_resident_counts(const nfx_solver* s, int64_t* h_counts);
 /* Give the solver a 3 x 3 block CSR copy of the FP32 operator it is then called with

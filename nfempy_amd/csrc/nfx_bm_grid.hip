@@ -32,8 +32,9 @@ constexpr int64_t kBmGridShare = 128 << 10;
 // launch) in 1 launch 12.6/35.1 | 5.1/15.1, in 2 24.1/39.2 | 9.7/16.5, in 3 35.9/42.4 | 14.6/18.4, in 4 46.4/45.6
 // | 19.2/19.6, in 6 68.5/64.9 | 28.4/25.9, in 12 137/98 | 56/43; of 5 cubed (15 blocks, 17 a launch) in 3
 // 19.7/26.6 | 12.9/17.1, in 6 38.8/43.7 | 25.3/26.7; of degree 1, 6 cubed (3 blocks) in 3 8.0/11.9 | 9.8/13.5.
+constexpr int kBmGridLaunches = 6;
 inline bool bm_grid_pays(int launches, int blocks, int cap) {
-  return launches <= 3 || (launches <= 6 && 4 * (int64_t)blocks >= 3 * (int64_t)launches * cap);
+  return launches <= 3 || (launches <= kBmGridLaunches && 4 * (int64_t)blocks >= 3 * (int64_t)launches * cap);
 }
 
 struct BmGridArgs {
@@ -580,10 +581,12 @@ static int bm_grid_plan(BmGrid* g, const std::vector<int>& rows, int64_t n_total
   NFX_CHECK_HIP(hipMemcpyAsync(nnz.data(), scratch, sizeof(int32_t) * n_inst, hipMemcpyDeviceToHost, st));
   NFX_CHECK_HIP(hipStreamSynchronize(st));
   std::vector<int> nblk(n_inst), order(n_inst);
+  int64_t total = 0;
   for (int i = 0; i < n_inst; ++i) {
     nblk[i] = bm_grid_blocks(rows[i], nnz[i]);
     order[i] = i;
-    if (nblk[i] < 1 || nblk[i] > cap) return NFX_OK;
+    total += nblk[i];
+    if (nblk[i] < 1 || nblk[i] > cap || total > (int64_t)kBmGridLaunches * cap) return NFX_OK;
   }
   std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return nblk[a] > nblk[b]; });
   std::vector<std::vector<BmGridBlock>> waves;

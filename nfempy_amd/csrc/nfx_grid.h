@@ -34,7 +34,7 @@ constexpr int kGridThreads = 1024;
 
 // A device gives the resources of cooperative launches to one process at a time; a launch in another is
 // refused, after ~35 ms. The callers then take the stepwise kernels, and for kGridRetrySeconds they do not
-// ask that device again (nfx_backoff.h); nor after a wait that was given up, for half a second.
+// ask that device again (nfx_backoff.h); nor after a launch whose blocks gave up waiting for each other.
 constexpr int kGridRetrySeconds = 10;
 
 // what a launch (or one system of it) reports

@@ -117,8 +117,8 @@ class MinresBatch:
     """Batched FP32 MINRES + FP64 refinement over independent systems (``nfx_minres_batch``):
     one set of launches per iteration for all instances (small batches: one launch per inner
     solve, ``set_resident``), each with its own recurrence, stopping test and refinement; on
-    either route an instance's result does not depend on the other instances. ``systems``: dicts with rowptr, col, vals32, vals64 and
-    optional sign / pinv (the symmetric form D A and a diagonal preconditioner)."""
+    either route an instance's result does not depend on the other instances. ``systems``:
+    dicts with rowptr, col, vals32, vals64 and optional sign / pinv (the symmetric form D A and a diagonal preconditioner)."""
 
     def __init__(self, systems, stream=None):
         self._systems = list(systems)
@@ -155,7 +155,8 @@ class MinresBatch:
         nat.call("nfx_minres_batch_set_resident", self._h, launches, int(absent))
 
     def resident_counts(self):
-        """Inner solves of instances that ran as one resident launch, and those that were tried so and ran stepwise."""
+        """Inner solves of instances that ran as one resident launch, and those that were tried so and ran
+        stepwise."""
         out = (ctypes.c_int64 * 2)()
         nat.call("nfx_minres_batch_resident_counts", self._h, out)
         return out[0], out[1]

@@ -390,10 +390,11 @@ def test_a_batch_keeps_one_route():
         one.close()
 
 
-@pytest.mark.parametrize("spec,count,resident", [((9, 2), 6, True), ((9, 2), 7, False), ((5, 2), 96, True)])
+@pytest.mark.parametrize("spec,count,resident", [((9, 2), 6, True), ((9, 2), 7, False), ((5, 2), 96, True),
+                                                 ((5, 2), 103, False)])
 def test_a_batch_is_resident_where_its_launches_pay(spec, count, resident):
     """Instances of 9 cubed of degree 2 take 87 blocks, two a launch of 256: three launches pay, four, two
-    thirds full, do not. Instances of 5 cubed take 15 blocks: six launches for 1,440 of them pay."""
+    thirds full, do not. Instances of 5 cubed take 15 blocks: six launches for 1,440 of them pay, 1,545 would be seven."""
     print(f"[routes] launches of {count}", flush=True)
     b, mb, rhs, _ = _batch([spec] * count)
     x, infos = mb.solve(rhs, rtol=1e-8)
